@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "common.cuh"
+#include "dense_common.cuh"
 #include "host_common.h"
 
 #pragma clang fp contract(off)
@@ -154,16 +155,6 @@ __global__ __launch_bounds__(256) void norm_rows_any_kernel(const T* __restrict_
   }
 }
 
-// out[r][i] = silu(gate[r][i]) * up[r][i] with gate_up = [rows][2*inter]
-// (gate columns, then up columns): silu(v) = v / (1 + exp(-v)) rounded per
-// op (exp, the sum, the quotient), then the product rounded.
-template <typename T>
-__device__ __forceinline__ float silu_mul_rounded(float g, float u) {
-  const float e = round_to<T>(expf(-g));
-  const float s = round_to<T>(g / round_to<T>(1.f + e));
-  return s * u;
-}
-
 template <typename T>
 __global__ void silu_mul_kernel(const T* __restrict__ gate_up, T* __restrict__ out, int inter) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
@@ -278,7 +269,8 @@ __global__ __launch_bounds__(64) void argmax_final_kernel(const T* __restrict__ 
 
 // ---------------------------------------------------------------------------
 // Decode-shaped linear layers on MFMA: y[rows][N] = x[rows][K] . W[N][K]^T for
-// rows <= 64 (one decode step's batch), bf16/f16 in, f32 accumulation.
+// rows <= 64 (one decode step's batch; more run on the tiled kernel of
+// dense_tile.hip), bf16/f16 in, f32 accumulation.
 //
 // Work split: workgroup (g, ks) owns FT tiles of 16 output features, the
 // whole batch and the ks-th of KS equal slices of K; its four waves split the
@@ -301,71 +293,6 @@ __global__ __launch_bounds__(64) void argmax_final_kernel(const T* __restrict__ 
 //   kEpiSiluMul   act = round(silu(round(gate)) * round(up)): tile i holds
 //                 gate rows 8i..8i+7 and up rows n1+8i..n1+8i+7
 // ---------------------------------------------------------------------------
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
-template <typename T>
-struct Mma16;
-template <>
-struct Mma16<bf16> {
-  static __device__ __forceinline__ f32x4_t run(u32x4_t a, u32x4_t b, f32x4_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-  }
-};
-template <>
-struct Mma16<f16> {
-  static __device__ __forceinline__ f32x4_t run(u32x4_t a, u32x4_t b, f32x4_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
-                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
-  }
-};
-// f32 (the reference CPU path's dtype): a 16-byte operand load holds four
-// floats, so a k step spans 16 elements, lane l holding elements
-// 4*(l/16) .. +3 of its row. v_mfma_f32_16x16x4_f32 number m takes each
-// lane's element m, for A and B alike: its four k indices are 4g + m over
-// the lane groups g, and the four products cover the step. The accumulator
-// layout is the 16-bit products' (lane l: D[4*(l/16) + v][l%16]).
-template <>
-struct Mma16<float> {
-  static __device__ __forceinline__ f32x4_t run(u32x4_t a, u32x4_t b, f32x4_t c) {
-#pragma unroll
-    for (int m = 0; m < 4; ++m)
-      c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[m]), __uint_as_float(b[m]), c, 0,
-                                               0, 0);
-    return c;
-  }
-};
-// Elements of one k step (four lanes groups' 16-byte loads) and of one
-// lane's load.
-template <typename T>
-__host__ __device__ constexpr int dense_step_elems() { return 64 / (int)sizeof(T); }
-
-enum : int { kEpiStore = 0, kEpiQkv = 1, kEpiResidual = 2, kEpiSiluMul = 3 };
-
-struct DenseParams {
-  const void* x;     // [rows][K]
-  const void* w;     // [N][K]
-  const void* bias;  // [N] or null (kEpiStore, kEpiQkv)
-  void* out0;        // y [rows][N] | q [rows][n1] | x_res [rows][N] | act [rows][n1]
-  void* out1;        // k [rows][n2 - n1] (kEpiQkv)
-  void* out2;        // v [rows][N - n2] (kEpiQkv)
-  // KS > 1: sticky error flags, one launch counter per wave slot
-  // (kDenseCtrWords) and (tile groups) x (KS - 1) records of FT*RT*256
-  // tagged 64-bit words.
-  uint32_t* ws_err;
-  uint32_t* ws_ctr;
-  uint64_t* ws_rec;
-  unsigned long long wait_ticks;
-  int rows, K, N, n1, n2;
-  int ksplit;        // KS
-  int steps;         // 32-wide k steps per wave
-  int packed;        // w in the tile order rlse_dense_pack writes
-  int xpacked;       // x in the packed row order (RLSE_PACKED_ROWS)
-  int opacked;       // kEpiSiluMul: act in the packed row order (RLSE_PACKED_OUT)
-};
-
 constexpr int kDenseWaves = 4;
 constexpr int kDenseMaxRows = 64;
 constexpr int kDenseMaxSplit = 8;
@@ -377,33 +304,6 @@ constexpr int kDenseMaxInner = 4;
 // when it has fewer than 256 tile groups, into ceil(256 / groups) slices.
 constexpr int kDenseCtrWords = 512 * kDenseWaves;
 constexpr int kDenseHeaderWords = 64;
-
-template <typename T>
-__device__ __forceinline__ void load4(const T* p, float* v) {
-  if constexpr (sizeof(T) == 4) {
-    const float4 u = *reinterpret_cast<const float4*>(p);
-    v[0] = u.x;
-    v[1] = u.y;
-    v[2] = u.z;
-    v[3] = u.w;
-  } else {
-    const uint2 u = *reinterpret_cast<const uint2*>(p);
-    const uint4 q = make_uint4(u.x, u.y, 0, 0);
-    float t[8];
-    Packet<T>::unpack(q, t);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = t[e];
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ void store4(T* p, const float* v) {
-  if constexpr (sizeof(T) == 4)
-    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-  else
-    *reinterpret_cast<uint2*>(p) = make_uint2(Packet<T>::pack2(v[0], v[1]),
-                                              Packet<T>::pack2(v[2], v[3]));
-}
 
 // KV > 1: the K split runs inside the workgroup instead of across
 // workgroups -- KV slices of kDenseWaves waves each, every wave on the k
@@ -718,8 +618,7 @@ bool aligned(const void* ptr, size_t a) { return ((uintptr_t)ptr % a) == 0; }
 // columns of its K range, so x costs (rows / (16 * tiles per group)) times
 // the weight bytes in L2 reads: lm_head-sized outputs take four tiles
 // (plain stores only); batches of more than 32 rows take two when the
-// output still has 256 groups of two, so no K split is needed (the rows of
-// the first 64-row chunk decide; every chunk uses the same grouping).
+// output still has 256 groups of two, so no K split is needed.
 // Measured at 64 rows: gate/up of 9728 x 896, 18.4 -> 16.0 us; for outputs
 // that then needed a K split (q/k/v 1152 x 896: 7.9 -> 11.6 us) two tiles
 // cost more than they saved.
@@ -745,17 +644,26 @@ int dense_split(int groups, int K) {
   return std::max(ks, 1);
 }
 
-// Launches dense_rows_kernel over the batch in chunks of kDenseMaxRows rows
-// (each chunk streams the weights once). Shapes were checked by the caller:
+// Whether more than kDenseMaxRows rows still run on dense_rows_kernel (a
+// split that fits in the workgroup, a row tile per workgroup row) instead of
+// the tiled kernel: products with a long K and few output tiles, whose K the
+// 16 waves of a workgroup stream faster than one tile's pipeline. Measured
+// (us, here / tiled): 1024 x 3072 at 128 rows 7.8 / 8.8, at 256 rows 13.6 /
+// 9.3; 896 x 4864 at 128 rows 9.4 / 12.1, at 256 rows 17.0 / 12.9; with K
+// 2048, 1024 features and 128 rows 9.2 / 7.8.
+bool dense_long_k(int groups, int rows, int K) {
+  return K >= 96 * 32 && groups * ((rows + 15) / 16) <= 512;
+}
+
+// Launches a product: dense_rows_kernel for a decode batch, the tiled kernel
+// for more rows. Shapes were checked by the caller:
 // K % 32 == 0, 16-feature tiles that never straddle an output, 16-byte
 // aligned x / W and 8-byte aligned outputs; ws holds ws_words words (zero
 // before the first launch; every launch leaves it zero).
 template <typename T, int EPI>
-int launch_dense(DenseParams p, size_t x_stride, size_t o0_stride, size_t o1_stride,
-                 size_t o2_stride, size_t ws_words, hipStream_t s) {
-  const int total_rows = p.rows;
+int launch_dense(DenseParams p, size_t ws_words, hipStream_t s) {
   const int tiles = EPI == kEpiSiluMul ? p.n1 / 8 : p.N / 16;
-  const int ft = dense_tiles_per_group(EPI == kEpiStore, total_rows, tiles);
+  const int ft = dense_tiles_per_group(EPI == kEpiStore, p.rows, tiles);
   const bool wide = ft == 4;
   const int groups = tiles / ft;
   const int ks = p.ws_rec ? dense_split(groups, p.K) : 1;
@@ -769,80 +677,71 @@ int launch_dense(DenseParams p, size_t x_stride, size_t o0_stride, size_t o1_str
   // registers per lane, so it keeps the split grid.
   const int kv_inner =
       (ks > 1 && ft == 1 && EPI != kEpiSiluMul &&
-       (total_rows <= 32 || EPI == kEpiResidual || EPI == kEpiQkv))
+       (p.rows <= 32 || EPI == kEpiResidual || EPI == kEpiQkv))
           ? std::min(ks, kDenseMaxInner)
           : 1;
+  if constexpr (EPI != kEpiStore) {  // plain stores come 64 rows at a time
+    if (p.rows > kDenseMaxRows && !(kv_inner > 1 && dense_long_k(groups, p.rows, p.K)))
+      return launch_dense_tile(EPI, std::is_same<T, bf16>::value ? RLSE_DTYPE_BF16 : RLSE_DTYPE_F16,
+                               p, s);
+  }
   const int ns = kv_inner > 1 ? kv_inner : ks;
   const int steps_total = p.K / dense_step_elems<T>();
   const int slice = (steps_total + ns - 1) / ns;
   p.ksplit = kv_inner > 1 ? 1 : ks;
   p.steps = (slice + kDenseWaves - 1) / kDenseWaves;
-  const char* base0 = (const char*)p.out0;
-  const char* base1 = (const char*)p.out1;
-  const char* base2 = (const char*)p.out2;
-  const char* xb = (const char*)p.x;
-  for (int r0 = 0; r0 < total_rows; r0 += kDenseMaxRows) {
-    DenseParams q = p;
-    q.rows = std::min(kDenseMaxRows, total_rows - r0);
-    q.x = xb + (size_t)r0 * x_stride * sizeof(T);
-    q.out0 = (void*)(base0 + (size_t)r0 * o0_stride * sizeof(T));
-    q.out1 = base1 ? (void*)(base1 + (size_t)r0 * o1_stride * sizeof(T)) : nullptr;
-    q.out2 = base2 ? (void*)(base2 + (size_t)r0 * o2_stride * sizeof(T)) : nullptr;
-    const int rt = (q.rows + 15) / 16;
-    if (q.ksplit > 1 && dense_ws_fixed_words() + (size_t)groups * (ks - 1) * ft * rt * 256 * 2 >
-                            ws_words)
-      return fail(RLSE_ERR_INVALID_VALUE, "dense: workspace too small");
-    if (q.ksplit > 1 && groups * ks * kDenseWaves > kDenseCtrWords)
-      return fail(RLSE_ERR_INVALID_VALUE, "dense: K-split grid larger than its counters");
-    const dim3 block(64 * kDenseWaves);
-    const dim3 grid(groups * q.ksplit);
-    auto run = [&](auto rt_c) {
-      constexpr int RT = decltype(rt_c)::value;
-      if constexpr ((RT <= 2 || EPI == kEpiResidual || EPI == kEpiQkv) && EPI != kEpiSiluMul) {
-        if (kv_inner > 1) {
-          // A residual or q/k/v projection's row tiles go to separate
-          // workgroups (grid rows): each streams the tile group's weights
-          // (the others from L2/MALL) but only its 16 rows of the batch's
-          // activations, which are most of a workgroup's bytes, and more
-          // compute units take part. Same k steps and sums per row, so the
-          // same bits. Measured in the whole decode step: o_proj and
-          // down_proj 8.05 -> 6.14 us at 32 rows x hidden 1024; at 64 rows
-          // x hidden 896, where it replaces the split grid's records, 11.86
-          // -> 6.46 us, and q/k/v 8.96 -> 6.27 us.
-          constexpr int RTL = (EPI == kEpiResidual || EPI == kEpiQkv) ? 1 : RT;
-          const dim3 g(grid.x, RT / RTL);
-          const dim3 big(64 * kDenseWaves * kv_inner);
-          if (kv_inner == 2)
-            hipLaunchKernelGGL((dense_rows_kernel<T, RTL, 1, EPI, 2>), g, big, 0, s, q);
-          else if (kv_inner == 3)
-            hipLaunchKernelGGL((dense_rows_kernel<T, RTL, 1, EPI, 3>), g, big, 0, s, q);
-          else
-            hipLaunchKernelGGL((dense_rows_kernel<T, RTL, 1, EPI, 4>), g, big, 0, s, q);
-          return;
-        }
-      }
-      if constexpr (EPI == kEpiStore) {
-        if (wide) {
-          hipLaunchKernelGGL((dense_rows_kernel<T, RT, 4, EPI>), grid, block, 0, s, q);
-          return;
-        }
-      }
-      if (ft == 2) {  // every chunk keeps the grouping (a short last chunk too)
-        hipLaunchKernelGGL((dense_rows_kernel<T, RT, 2, EPI>), grid, block, 0, s, q);
+  const int rt = (p.rows + 15) / 16;
+  if (p.ksplit > 1 && dense_ws_fixed_words() + (size_t)groups * (ks - 1) * ft * rt * 256 * 2 >
+                          ws_words)
+    return fail(RLSE_ERR_INVALID_VALUE, "dense: workspace too small");
+  if (p.ksplit > 1 && groups * ks * kDenseWaves > kDenseCtrWords)
+    return fail(RLSE_ERR_INVALID_VALUE, "dense: K-split grid larger than its counters");
+  const dim3 block(64 * kDenseWaves);
+  const dim3 grid(groups * p.ksplit);
+  auto run = [&](auto rt_c) {
+    constexpr int RT = decltype(rt_c)::value;
+    if constexpr ((RT <= 2 || EPI == kEpiResidual || EPI == kEpiQkv) && EPI != kEpiSiluMul) {
+      if (kv_inner > 1) {
+        // A residual or q/k/v projection's row tiles go to separate
+        // workgroups (grid rows): each streams the tile group's weights
+        // (the others from L2/MALL) but only its 16 rows of the batch's
+        // activations, which are most of a workgroup's bytes, and more
+        // compute units take part. Same k steps and sums per row, so the
+        // same bits. Measured in the whole decode step: o_proj and
+        // down_proj 8.05 -> 6.14 us at 32 rows x hidden 1024; at 64 rows
+        // x hidden 896, where it replaces the split grid's records, 11.86
+        // -> 6.46 us, and q/k/v 8.96 -> 6.27 us.
+        constexpr int RTL = (EPI == kEpiResidual || EPI == kEpiQkv) ? 1 : RT;
+        const dim3 g(grid.x, RTL < RT || p.rows > kDenseMaxRows ? rt : 1);
+        const dim3 big(64 * kDenseWaves * kv_inner);
+        if (kv_inner == 2)
+          hipLaunchKernelGGL((dense_rows_kernel<T, RTL, 1, EPI, 2>), g, big, 0, s, p);
+        else if (kv_inner == 3)
+          hipLaunchKernelGGL((dense_rows_kernel<T, RTL, 1, EPI, 3>), g, big, 0, s, p);
+        else
+          hipLaunchKernelGGL((dense_rows_kernel<T, RTL, 1, EPI, 4>), g, big, 0, s, p);
         return;
       }
-      hipLaunchKernelGGL((dense_rows_kernel<T, RT, 1, EPI>), grid, block, 0, s, q);
-    };
-    switch (rt) {
-      case 1: run(std::integral_constant<int, 1>{}); break;
-      case 2: run(std::integral_constant<int, 2>{}); break;
-      case 3: run(std::integral_constant<int, 3>{}); break;
-      default: run(std::integral_constant<int, 4>{}); break;
     }
-    const int rc = launch_status("dense_rows_kernel");
-    if (rc) return rc;
+    if constexpr (EPI == kEpiStore) {
+      if (wide) {
+        hipLaunchKernelGGL((dense_rows_kernel<T, RT, 4, EPI>), grid, block, 0, s, p);
+        return;
+      }
+    }
+    if (ft == 2) {
+      hipLaunchKernelGGL((dense_rows_kernel<T, RT, 2, EPI>), grid, block, 0, s, p);
+      return;
+    }
+    hipLaunchKernelGGL((dense_rows_kernel<T, RT, 1, EPI>), grid, block, 0, s, p);
+  };
+  switch (rt) {
+    case 1: run(std::integral_constant<int, 1>{}); break;
+    case 2: run(std::integral_constant<int, 2>{}); break;
+    case 3: run(std::integral_constant<int, 3>{}); break;
+    default: run(std::integral_constant<int, 4>{}); break;
   }
-  return RLSE_OK;
+  return launch_status("dense_rows_kernel");
 }
 
 // Workspace words a fused projection needs for its K split (0: none): the
@@ -880,10 +779,9 @@ int check_dense(const char* what, int dtype, int rows, int K, const void* x, con
 }
 
 template <int EPI>
-int dense_by_dtype(int dtype, const DenseParams& p, size_t xs, size_t s0, size_t s1, size_t s2,
-                   size_t ws_words, hipStream_t s) {
-  return dtype == RLSE_DTYPE_BF16 ? launch_dense<bf16, EPI>(p, xs, s0, s1, s2, ws_words, s)
-                                  : launch_dense<f16, EPI>(p, xs, s0, s1, s2, ws_words, s);
+int dense_by_dtype(int dtype, const DenseParams& p, size_t ws_words, hipStream_t s) {
+  return dtype == RLSE_DTYPE_BF16 ? launch_dense<bf16, EPI>(p, ws_words, s)
+                                  : launch_dense<f16, EPI>(p, ws_words, s);
 }
 
 // The caller's workspace for a fused projection: NULL runs without a K
@@ -1086,7 +984,7 @@ extern "C" int rlse_linear(const void* x, const void* weight, const void* bias, 
     p.rows = rows;
     p.K = in_features;
     p.N = out_features;
-    return launch_dense<float, kEpiStore>(p, in_features, out_features, 0, 0, 0, s);
+    return launch_dense<float, kEpiStore>(p, 0, s);
   }
   if (packed && !mfma)
     return fail(RLSE_ERR_INVALID_VALUE,
@@ -1107,7 +1005,16 @@ extern "C" int rlse_linear(const void* x, const void* weight, const void* bias, 
     p.N = out_features;
     p.packed = flags.packed;
     p.xpacked = flags.xpacked;
-    return dense_by_dtype<kEpiStore>(dtype, p, in_features, out_features, 0, 0, 0, s);
+    // 64 rows at a time: a row's bits do not depend on its neighbours.
+    for (int r0 = 0; r0 < rows; r0 += kDenseMaxRows) {
+      DenseParams q = p;
+      q.rows = std::min(kDenseMaxRows, rows - r0);
+      q.x = (const uint16_t*)x + (size_t)r0 * in_features;
+      q.out0 = (uint16_t*)y + (size_t)r0 * out_features;
+      const int rc = dense_by_dtype<kEpiStore>(dtype, q, 0, s);
+      if (rc) return rc;
+    }
+    return RLSE_OK;
   }
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
@@ -1183,8 +1090,7 @@ extern "C" int rlse_qkv_proj(const void* x, const void* w_qkv, const void* b_qkv
   size_t words = 0;
   rc = dense_workspace("qkv_proj", p, workspace, workspace_bytes, &words);
   if (rc) return rc;
-  return dense_by_dtype<kEpiQkv>(dtype, p, hidden, q_features, kv_features, kv_features, words,
-                                 as_stream(stream));
+  return dense_by_dtype<kEpiQkv>(dtype, p, words, as_stream(stream));
 }
 
 extern "C" int rlse_linear_residual(const void* x, const void* weight, void* residual, int rows,
@@ -1212,8 +1118,7 @@ extern "C" int rlse_linear_residual(const void* x, const void* weight, void* res
   size_t words = 0;
   rc = dense_workspace("linear_residual", p, workspace, workspace_bytes, &words);
   if (rc) return rc;
-  return dense_by_dtype<kEpiResidual>(dtype, p, in_features, out_features, 0, 0, words,
-                                      as_stream(stream));
+  return dense_by_dtype<kEpiResidual>(dtype, p, words, as_stream(stream));
 }
 
 extern "C" int rlse_gate_up_silu(const void* x, const void* w_gate_up, void* act, int rows,
@@ -1245,7 +1150,7 @@ extern "C" int rlse_gate_up_silu(const void* x, const void* w_gate_up, void* act
   size_t words = 0;
   rc = dense_workspace("gate_up_silu", p, workspace, workspace_bytes, &words);
   if (rc) return rc;
-  return dense_by_dtype<kEpiSiluMul>(dtype, p, hidden, inter, 0, 0, words, as_stream(stream));
+  return dense_by_dtype<kEpiSiluMul>(dtype, p, words, as_stream(stream));
 }
 
 extern "C" int rlse_dense_pack(const void* weight, void* packed, int out_features,

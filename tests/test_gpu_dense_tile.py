@@ -1,0 +1,109 @@
+"""The fused projections over more rows than a decode batch (prompts).
+
+Reference: the q/k/v, o, gate/up and down projections of the prefill branch
+(src/backends/qwen2.rs:153-175, 233-252). Shapes put the output on each tile
+size and on its edges: one row past a 16-row tile, features that end inside a
+tile, one, an odd number and an even number of 32-element k steps. The bar is
+one rounding of the dtype at the result's magnitude: the products are
+accumulated in f32, so a sum in another order moves a result by at most a
+neighbouring value, and each further rounding (the residual sum, silu's) by
+one more.
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from gpu_helpers import DEV
+
+pytestmark = pytest.mark.gpu
+
+_T = {"bf16": torch.bfloat16, "f16": torch.float16}
+ULP = {"bf16": 2.0 ** -7, "f16": 2.0 ** -10}
+# rows, hidden (K of q/k/v and gate/up), q features, kv features, inter
+SHAPES = [(65, 32, 32, 16, 32),        # 32 x 32 tiles, one k step
+          (81, 96, 64, 16, 32),        # three k steps
+          (129, 896, 896, 128, 1024),  # 64 x 64 tiles, q/k/v ends inside one
+          (337, 1024, 2048, 1024, 3104),  # 128 x 64 tiles, K 3104: 97 k steps
+          (97, 3072, 512, 256, 64)]    # a long K: row tiles per workgroup row
+
+
+def _dev(a, dt):
+    return torch.from_numpy(np.ascontiguousarray(a, np.float32)).to(DEV).to(_T[dt])
+
+
+def _pack_rows(x):
+    """[rows][K] -> packed rows, whole 16-row tiles."""
+    n, k = x.shape
+    full = np.zeros(((n + 15) // 16 * 16, k), np.float32)
+    full[:n] = x
+    return full.reshape(-1, 16, k // 32, 4, 8).transpose(0, 2, 3, 1, 4).reshape(full.shape)
+
+
+def _unpack_rows(x, n):
+    t, k = x.shape
+    return x.reshape(t // 16, k // 32, 4, 16, 8).transpose(0, 3, 1, 2, 4).reshape(t, k)[:n]
+
+
+def _close(name, got, want, dt, roundings):
+    torch.cuda.synchronize()
+    got = got.float().cpu().numpy() if isinstance(got, torch.Tensor) else got
+    scale = np.maximum(np.abs(want), np.sqrt(np.mean(want.astype(np.float64) ** 2)))
+    worst = float((np.abs(got - want) / (ULP[dt] * scale)).max())
+    print(f"[{name}] dtype={dt} worst {worst:.2f} of {roundings} ulps")
+    assert np.isfinite(got).all() and worst <= roundings, (name, worst)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("rows,hidden,nq,nkv,inter", SHAPES)
+def test_prompt_projections_match_oracle(kv, dt, packed, rows, hidden, nq, nkv, inter):
+    rng = np.random.default_rng(rows + hidden)
+    r = lambda *s: O.round_to(rng.standard_normal(s) / np.sqrt(s[-1]), dt)  # noqa: E731
+    tiles = (rows + 15) // 16 * 16
+    x = O.round_to(rng.standard_normal((rows, hidden)), dt)
+
+    def weight(w, pair=0):
+        w = _dev(w, dt)
+        if not packed:
+            return w
+        out = torch.empty_like(w)
+        kv.dense_pack(w, out, w.shape[0], w.shape[1], pair, dt)
+        return out
+
+    def ws(n_out, n_in):
+        n = kv.dense_workspace_size(rows, n_out, n_in)
+        return torch.zeros(max(n, 4), dtype=torch.uint8, device=DEV)
+
+    xd = _dev(_pack_rows(x) if packed else x, dt)
+    # guard rows past the outputs stay untouched
+    z = lambda n, extra=3: torch.full((rows + extra, n), 7.0, dtype=_T[dt], device=DEV)  # noqa: E731
+
+    wq = [r(n, hidden) for n in (nq, nkv, nkv)]
+    bq = [O.round_to(rng.standard_normal(n), dt) for n in (nq, nkv, nkv)]
+    outs = [z(n) for n in (nq, nkv, nkv)]
+    kv.qkv_proj(xd, weight(np.concatenate(wq)), _dev(np.concatenate(bq), dt), *outs, rows, hidden,
+                nq, nkv, dt, ws(nq + 2 * nkv, hidden), packed=packed, packed_x=packed)
+    for name, o, w, b in zip("qkv", outs, wq, bq):
+        _close(f"qkv_proj {name}", o[:rows], O.linear_ref(x, w, b, dt), dt, 2)
+        assert bool((o[rows:] == 7).all())
+
+    wg, wu = r(inter, hidden), r(inter, hidden)
+    act = torch.zeros((tiles, inter), dtype=_T[dt], device=DEV)
+    kv.gate_up_silu(xd, weight(np.concatenate([wg, wu]), inter), act, rows, hidden, inter, dt,
+                    ws(2 * inter, hidden), packed=packed, packed_x=packed, packed_out=packed)
+    want = O.silu_mul_ref(O.linear_ref(x, wg, None, dt), O.linear_ref(x, wu, None, dt), dt)
+    got = act.float().cpu().numpy()
+    # gate, up, exp, sum, quotient and product each round once
+    _close("gate_up_silu", _unpack_rows(got, rows) if packed else got[:rows], want, dt, 6)
+
+    if hidden % 16 == 0:
+        a = O.round_to(rng.standard_normal((rows, inter)), dt)
+        wd, res = r(hidden, inter), O.round_to(rng.standard_normal((rows, hidden)), dt)
+        y = z(hidden)
+        y[:rows] = _dev(res, dt)
+        kv.linear_residual(_dev(_pack_rows(a) if packed else a, dt), weight(wd), y, rows, hidden,
+                           inter, dt, ws(hidden, inter), packed=packed, packed_x=packed)
+        want = O.round_to(res + O.linear_ref(a, wd, None, dt), dt)
+        _close("linear_residual", y[:rows], want, dt, 2)
+        assert bool((y[rows:] == 7).all())
