@@ -7,6 +7,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "rlse_kv.h"
 
 namespace rlse {
@@ -80,6 +82,18 @@ __device__ __forceinline__ float add_rn(float a, float b) {
 template <typename T>
 __device__ __forceinline__ float round_to(float v) {
   return Elem<T>::to_f32(Elem<T>::from_f32(v));
+}
+
+// round_to through the conversion instruction: the same bits for every input
+// (NaNs included) without the integer sequence of f32_to_bf16_bits.
+template <typename T>
+__device__ __forceinline__ float round_cvt(float v) {
+  if constexpr (sizeof(T) == 4)
+    return v;
+  else if constexpr (std::is_same<T, bf16>::value)
+    return (float)(__bf16)v;
+  else
+    return (float)(f16)v;
 }
 
 // ---------------------------------------------------------------------------
@@ -170,6 +184,18 @@ struct Packet<f16> {
     return c;
   }
 };
+
+// A 16-byte packet of T from floats (round to nearest even).
+template <typename T>
+__device__ __forceinline__ uint4 cvt_packet(const float* v) {
+  if constexpr (sizeof(T) == 4) {
+    return make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]),
+                      __float_as_uint(v[3]));
+  } else {
+    return make_uint4(Packet<T>::pack2(v[0], v[1]), Packet<T>::pack2(v[2], v[3]),
+                      Packet<T>::pack2(v[4], v[5]), Packet<T>::pack2(v[6], v[7]));
+  }
+}
 
 // ---------------------------------------------------------------------------
 // Wave64 reductions. DPP controls (GCN/CDNA encoding): quad_perm [1,0,3,2]

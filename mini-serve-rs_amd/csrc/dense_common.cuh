@@ -2,8 +2,6 @@
 // instructions, a launch's parameters, the epilogues and four-element packets.
 #pragma once
 
-#include <type_traits>
-
 #include "common.cuh"
 
 namespace rlse {
@@ -98,18 +96,6 @@ __device__ __forceinline__ void store4(T* p, const float* v) {
   else
     *reinterpret_cast<uint2*>(p) = make_uint2(Packet<T>::pack2(v[0], v[1]),
                                               Packet<T>::pack2(v[2], v[3]));
-}
-
-// round_to through the conversion instruction (the same rounding; a NaN comes
-// out quiet).
-template <typename T>
-__device__ __forceinline__ float round_cvt(float v) {
-  if constexpr (sizeof(T) == 4)
-    return v;
-  else if constexpr (std::is_same<T, bf16>::value)
-    return (float)(__bf16)v;
-  else
-    return (float)(f16)v;
 }
 
 // out[r][i] = silu(gate[r][i]) * up[r][i] with gate_up = [rows][2*inter]

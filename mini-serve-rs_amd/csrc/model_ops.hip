@@ -39,18 +39,6 @@ __global__ void embedding_kernel(const int32_t* __restrict__ ids, const T* __res
     dst[c] = ok ? src[c] : make_uint4(0, 0, 0, 0);
 }
 
-// 16-byte packets of T as floats and back (round to nearest even).
-template <typename T>
-__device__ __forceinline__ uint4 pack_packet(const float* v) {
-  if constexpr (sizeof(T) == 4) {
-    return make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]),
-                      __float_as_uint(v[3]));
-  } else {
-    return make_uint4(Packet<T>::pack2(v[0], v[1]), Packet<T>::pack2(v[2], v[3]),
-                      Packet<T>::pack2(v[4], v[5]), Packet<T>::pack2(v[6], v[7]));
-  }
-}
-
 // Sum over a workgroup of kThreads threads, the same order in every thread.
 template <int kThreads>
 __device__ __forceinline__ float block_sum(float v, float* s_part) {
@@ -98,7 +86,7 @@ __global__ __launch_bounds__(kNormThreads) void norm_rows_kernel(
         Packet<T>::unpack(reinterpret_cast<const uint4*>(x + base)[ci], xv);
 #pragma unroll
         for (int e = 0; e < E; ++e) h[c][e] = round_to<T>(h[c][e] + xv[e]);
-        reinterpret_cast<uint4*>(residual + base)[ci] = pack_packet<T>(h[c]);
+        reinterpret_cast<uint4*>(residual + base)[ci] = cvt_packet<T>(h[c]);
       }
 #pragma unroll
       for (int e = 0; e < E; ++e) ss += h[c][e] * h[c][e];
@@ -120,7 +108,7 @@ __global__ __launch_bounds__(kNormThreads) void norm_rows_kernel(
           packed_out ? (((size_t)(blockIdx.x >> 4) * (n >> 5) + (ci >> 2)) * 64 + (blockIdx.x & 15) +
                         16 * (ci & 3)) * 8
                      : base + (size_t)ci * E;
-      *reinterpret_cast<uint4*>(out + at) = pack_packet<T>(o);
+      *reinterpret_cast<uint4*>(out + at) = cvt_packet<T>(o);
     }
   }
 }

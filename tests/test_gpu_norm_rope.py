@@ -148,3 +148,47 @@ def test_qwen2_path_without_qk_norm(kv):
     pool_k = to_host(kp)
     for i in range(b):
         np.testing.assert_array_equal(pool_k[tables[i, pos[i] // 16], :, pos[i] % 16], k_ref[i])
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("hq,hkv,d", [(7, 1, 64), (4, 2, 128), (3, 3, 32), (2, 1, 256)])
+@pytest.mark.parametrize("norm", [True, False])
+def test_qk_norm_rope_append_packet_rows_give_the_element_bits(kv, dtype, hq, hkv, d, norm):
+    """Aligned rows of whole packets (several rows a wave) and the same rows
+    one element into their buffers (a wave a row, element accesses) leave the
+    same bits: q, the appended K and V, and nothing where a position, page id
+    or sequence is invalid. NaN, infinities, zeros and subnormals included."""
+    g = torch.Generator(device=DEV).manual_seed(d + hq)
+    tdt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[dtype]
+    n, nb, mbps, max_pos = 37, 15, 5, 70
+    rnd = lambda *s: torch.randn(s, generator=g, device=DEV).to(tdt)  # noqa: E731
+    q, k, v = rnd(n, hq, d), rnd(n, hkv, d), rnd(n, hkv, d)
+    q[1, 0, 3], q[2, 0, d - 1], k[3, 0, 0], k[4, 0, 1] = float("inf"), float("nan"), -0.0, 1e-7
+    q[5], k[6] = 0.0, 3.0e4
+    w = [1 + 0.1 * rnd(d), 1 + 0.1 * rnd(d)] if norm else [None, None]
+    cos, sin = rnd(max_pos, d // 2), rnd(max_pos, d // 2)
+    pos = torch.arange(n, dtype=torch.int32, device=DEV)
+    pos[7], pos[8] = -1, max_pos
+    seq = (pos % 3).to(torch.int32)
+    seq[10], seq[11] = 3, -1
+    tables = torch.randperm(nb, generator=g, device=DEV).to(torch.int32).view(3, 5)
+    tables[0, 1], tables[1, 0] = nb, -1
+
+    def shifted(t, by):
+        buf = torch.full((t.numel() + 8,), 5.0, dtype=tdt, device=DEV)
+        out = buf[by:by + t.numel()].view(t.shape)
+        out.copy_(t)
+        return out
+
+    got = []
+    for by in (0, 1):
+        a = [None if t is None else shifted(t, by) for t in (q, k, v, *w, cos, sin)]
+        q_out, kp, vp = (shifted(torch.full(s, 9.0, dtype=tdt, device=DEV), by)
+                         for s in ((n, hq, d), (nb, hkv, 16, d), (nb, hkv, 16, d)))
+        kv.qk_norm_rope_append(*a[:5], 1e-6, *a[5:], max_pos, pos, tables, 3, seq, n, hq, hkv, d,
+                               mbps, nb, q_out, kp, vp, dtype)
+        torch.cuda.synchronize()
+        got.append([t.contiguous().view(torch.int32 if dtype == "f32" else torch.int16).cpu()
+                    for t in (q_out, kp, vp)])
+    for x, y in zip(*got):
+        assert torch.equal(x, y)
