@@ -30,16 +30,6 @@ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
   return (uint16_t)(u >> 16);
 }
 
-// The same rounding with the NaN test as a select (v_cndmask) instead of an
-// exec-masked branch: cheaper in straight-line element-wise code, at the cost
-// of a few live registers.
-__device__ __forceinline__ uint16_t f32_to_bf16_bits_sel(float f) {
-  const uint32_t u = __float_as_uint(f);
-  const uint32_t rne = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
-  const uint32_t qnan = (u >> 16) | 0x40u;
-  return (uint16_t)(((u & 0x7fffffffu) > 0x7f800000u) ? qnan : rne);
-}
-
 template <typename T>
 struct Elem;
 

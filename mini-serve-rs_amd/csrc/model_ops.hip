@@ -85,7 +85,7 @@ __global__ __launch_bounds__(kNormThreads) void norm_rows_kernel(
         float xv[E];
         Packet<T>::unpack(reinterpret_cast<const uint4*>(x + base)[ci], xv);
 #pragma unroll
-        for (int e = 0; e < E; ++e) h[c][e] = round_to<T>(h[c][e] + xv[e]);
+        for (int e = 0; e < E; ++e) h[c][e] = round_cvt<T>(h[c][e] + xv[e]);
         reinterpret_cast<uint4*>(residual + base)[ci] = cvt_packet<T>(h[c]);
       }
 #pragma unroll
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kNormThreads) void norm_rows_kernel(
       float wv[E], o[E];
       Packet<T>::unpack(wp[c], wv);
 #pragma unroll
-      for (int e = 0; e < E; ++e) o[e] = round_to<T>(h[c][e] / norm) * wv[e];
+      for (int e = 0; e < E; ++e) o[e] = round_cvt<T>(h[c][e] / norm) * wv[e];
       // Packed rows (16-bit): row r's packet ci (elements 8ci .. +8) goes to
       // ((r/16 * n/32 + ci/4) * 64 + r%16 + 16 (ci%4)) * 8, the order in
       // which dense_rows_kernel loads its B operands.
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(256) void norm_rows_any_kernel(const T* __restrict_
   for (int i = lane; i < n; i += 64) {
     float h = Elem<T>::to_f32(rr[i]);
     if constexpr (ADD) {
-      h = round_to<T>(h + Elem<T>::to_f32(x[row * n + i]));
+      h = round_cvt<T>(h + Elem<T>::to_f32(x[row * n + i]));
       rr[i] = Elem<T>::from_f32(h);
     }
     ss += h * h;
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(256) void norm_rows_any_kernel(const T* __restrict_
   ss = wave_sum(ss);
   const float norm = sqrtf(ss * inv_n + eps);
   for (int i = lane; i < n; i += 64) {
-    const float xn = round_to<T>(Elem<T>::to_f32(rr[i]) / norm);
+    const float xn = round_cvt<T>(Elem<T>::to_f32(rr[i]) / norm);
     orow[i] = Elem<T>::from_f32(xn * Elem<T>::to_f32(w[i]));
   }
 }
@@ -553,7 +553,7 @@ __global__ __launch_bounds__(64 * kDenseWaves * KV) void dense_rows_kernel(Dense
     if constexpr (EPI == kEpiSiluMul) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        o[e] = ok ? silu_mul_rounded<T>(round_to<T>(v[k][0][e]), round_to<T>(v[k][1][e]))
+        o[e] = ok ? silu_mul_rounded<T>(round_cvt<T>(v[k][0][e]), round_cvt<T>(v[k][1][e]))
                   : __builtin_nanf("");
       const int c = tile * 8 + fq;  // act feature (4 of them)
       store4<T>((T*)p.out0 +
@@ -564,13 +564,13 @@ __global__ __launch_bounds__(64 * kDenseWaves * KV) void dense_rows_kernel(Dense
     } else if constexpr (EPI == kEpiResidual) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        o[e] = ok ? pre[k][e] + round_to<T>(v[k][0][e]) : __builtin_nanf("");
+        o[e] = ok ? pre[k][e] + round_cvt<T>(v[k][0][e]) : __builtin_nanf("");
       store4<T>((T*)p.out0 + (size_t)b * p.N + tile * 16 + fq, o);
     } else {
       const int n = tile * 16 + fq;
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        o[e] = ok ? round_to<T>(v[k][0][e]) + (p.bias ? pre[k][e] : 0.f) : __builtin_nanf("");
+        o[e] = ok ? round_cvt<T>(v[k][0][e]) + (p.bias ? pre[k][e] : 0.f) : __builtin_nanf("");
       T* dst;
       if (EPI == kEpiQkv && n >= p.n2)
         dst = (T*)p.out2 + (size_t)b * (p.N - p.n2) + (n - p.n2);
