@@ -35,6 +35,7 @@
 // of the four key rows -- four consecutive keys of one dimension.
 #include <math.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "common.cuh"
@@ -61,8 +62,7 @@ constexpr int kBN = 64;            // keys per tile
 // cycles per read.)
 constexpr int kPadK = 8;
 constexpr int kPadV = 32;
-constexpr int kMinKeysPerSplit = 512;
-constexpr int kMaxSplits = 16;
+constexpr int kMaxSplits = 32;
 constexpr int kMaxSplitPages = 1024;  // page ids of a split staged in LDS (16384 keys)
 // The running max of a query's softmax moves only when a score exceeds it by
 // more than this many powers of two (probabilities stay below 2^kLazyLog2).
@@ -114,7 +114,11 @@ __device__ __forceinline__ float4* part_block(const PrefillParams& p, int sp, in
   return reinterpret_cast<float4*>(p.part) + wgi * (4 * (D / 32) + 1) * kPThreads;
 }
 
-template <typename T, int D>
+// FEW: a chunk too short to give every wave of the one row tile rows; the
+// waves without any then only stage. (Left out otherwise: the branch around
+// the math costs the full kernel 3-9%; with 5 tokens of a group of 4 it takes
+// 8000 cached keys from 28.6 to 21.7 us.)
+template <typename T, int D, bool FEW>
 __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) {
   constexpr int KB = D / 16;                  // 16-wide k-blocks of q.k
   constexpr int DB = D / 32;                  // 32-row blocks of O^T
@@ -145,6 +149,7 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
   const int myrow = rt * kBM + wave * 32 + col;
   const int row_c = myrow < rows ? myrow : rows - 1;
   const int t = row_c / G, g = row_c - t * G, qh = h * G + g;
+  const bool live = rt * kBM + wave * 32 < rows;  // the wave has rows (else it only stages)
   const int kmax = p.offset + t;  // last key this query sees
   // Last key every query of this wave sees (its first row has the smallest t).
   const int kmin_wave = p.offset + min(rt * kBM + wave * 32, rows - 1) / G;
@@ -251,6 +256,7 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
       load_tile(more ? kt + kBN : kt);  // in flight during this tile's math
       const int vbits = s_valid[bf];
 
+      if (!FEW || live) {
       // S^T for the two 32-key halves of the tile.
       // (The two halves' MFMA chains are interleaved: consecutive MFMAs then
       // never wait on each other's accumulator.)
@@ -331,6 +337,7 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
           const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
           o[db] = Mfma<T>::mma(make_uint4(l2.x, l2.y, h2.x, h2.y), pk[kq], o[db]);
         }
+      }
 
       if (!more) break;
       store_tile(bf ^ 1);
@@ -362,6 +369,7 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
   // blk + (k*kPThreads + tid)*4 floats, slots 0..4*DB-1 holding acc and slot 4*DB
   // (m, l) -- so every store covers 1 KB of consecutive bytes. The merge
   // launch reads them back with the same thread-to-row map.
+  if (!live) return;  // the merge reads no row of this wave
   float4* blk = part_block<D>(p, split, h, rt) + tid;
 #pragma unroll
   for (int db = 0; db < DB; ++db)
@@ -391,7 +399,7 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
 // 32 banks apart.
 constexpr int kPadF = 4;
 constexpr int kPadFV = 8;
-template <int D>
+template <int D, bool FEW>
 __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel_f32(PrefillParams p) {
   constexpr int DB = D / 32;                  // 32-row blocks of O^T
   constexpr int KH = D / 2;                   // k steps of q.k
@@ -421,6 +429,7 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel_f32(PrefillParams
   const int myrow = rt * kBM + wave * 32 + col;
   const int row_c = myrow < rows ? myrow : rows - 1;
   const int t = row_c / G, g = row_c - t * G, qh = h * G + g;
+  const bool live = rt * kBM + wave * 32 < rows;
   const int kmax = p.offset + t;
   const int kmin_wave = p.offset + min(rt * kBM + wave * 32, rows - 1) / G;
   const int last_row = min(rows - 1, rt * kBM + kBM - 1);
@@ -513,6 +522,7 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel_f32(PrefillParams
       load_tile(more ? kt + kBN : kt);  // in flight during this tile's math
       const int vbits = s_valid[bf];
 
+      if (!FEW || live) {
       f32x16_t s[2];
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb)
@@ -577,6 +587,7 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel_f32(PrefillParams
           for (int db = 0; db < DB; ++db)
             o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[db * 32], s[sb][j], o[db], 0, 0, 0);
         }
+      }
 
       if (!more) break;
       store_tile(bf ^ 1);
@@ -601,6 +612,7 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel_f32(PrefillParams
     return;
   }
   // Key splits: the partial block in the 16-bit kernel's layout.
+  if (!live) return;  // the merge reads no row of this wave
   float4* blk = part_block<D>(p, split, h, rt) + tid;
 #pragma unroll
   for (int db = 0; db < DB; ++db)
@@ -692,38 +704,58 @@ struct PrefillPlan {
   size_t ws_bytes;
 };
 
-int plan_prefill(int Tq, int ctx_len, int Hq, int Hkv, int D, PrefillPlan* plan) {
+// Splits of the keys: the count with the least estimated time, in us,
+//   rounds of workgroups over the compute units x tiles per split x t
+//   + (more than one split) the merge launch, a round trip per kMergeBatch
+//     splits and the partial blocks written and read back.
+// t is a tile's time in a workgroup, measured on one split of long contexts.
+// Measured against one workgroup per compute unit with at least 512 keys
+// each: f32, 16/8 heads of 128, 333 tokens after 1030: 8 splits for 3, 135 ->
+// 68 us; 20 tokens after 1030: 17 for 3, 97 -> 32 us; bf16, 14/2 heads of 64,
+// 2000 tokens: 2 for 3 (one round for two), 36 -> 33 us.
+int plan_prefill(int Tq, int ctx_len, int Hq, int Hkv, int D, int dtype, PrefillPlan* plan) {
   int cus = 0;
   const int st = device_cu_count(&cus);
   if (st) return st;
   const int G = Hq / Hkv;
   plan->row_tiles = (Tq * G + kBM - 1) / kBM;
   const long long base = (long long)plan->row_tiles * Hkv;
-  int s = (int)(((long long)cus + base - 1) / base);  // one group per compute unit
-  const int by_len = (ctx_len + kMinKeysPerSplit - 1) / kMinKeysPerSplit;
-  s = s < by_len ? s : by_len;
-  s = s < kMaxSplits ? s : kMaxSplits;
-  const int by_pages = (ctx_len + kMaxSplitPages * 16 - 1) / (kMaxSplitPages * 16);
-  s = s > by_pages ? s : by_pages;  // a split's page ids must fit the LDS stage
-  s = s < 1 ? 1 : s;
-  int per = (ctx_len + s - 1) / s;
-  per = (per + kBN - 1) / kBN * kBN;
-  s = (ctx_len + per - 1) / per;  // drop splits left empty by the rounding
-  plan->splits = s;
-  plan->split_keys = per;
-  plan->ws_bytes = s > 1 ? (size_t)s * Hkv * plan->row_tiles * (4 * (D / 32) + 1) * kPThreads *
-                               4 * sizeof(float)
-                         : 0;
+  const size_t block = (size_t)(4 * (D / 32) + 1) * kPThreads * 4 * sizeof(float);
+  const double tile_us = dtype == RLSE_DTYPE_F32 ? (D == 128 ? 14.7 : 7.7) : (D == 128 ? 1.9 : 1.2);
+  const int tiles = (ctx_len + kBN - 1) / kBN;
+  const int most = kMaxSplitPages * 16 / kBN;  // a split's page ids must fit the LDS stage
+  const int limit = std::min(tiles, std::max(kMaxSplits, (tiles + most - 1) / most));
+  int best = 0, best_per = 0;
+  double best_us = 0.;
+  for (int want = 1; want <= limit; ++want) {
+    const int per = (tiles + want - 1) / want, s = (tiles + per - 1) / per;
+    if (s != want || per > most) continue;  // (fewer splits gave the same shares)
+    double us = (double)((base * s + cus - 1) / cus) * per * tile_us;
+    if (s > 1) us += 3. + 1.5 * ((s + kMergeBatch - 1) / kMergeBatch) + 2. * base * s * block / 4e6;
+    if (best == 0 || us < best_us) best = s, best_per = per, best_us = us;
+  }
+  plan->splits = best;
+  plan->split_keys = best_per * kBN;
+  plan->ws_bytes = best > 1 ? (size_t)best * base * block : 0;
   return RLSE_OK;
 }
 
 template <typename T, int D>
 int launch_prefill(PrefillParams& pp, hipStream_t stream) {
   const int nwg = pp.row_tiles * pp.Hkv * pp.splits;
-  if constexpr (sizeof(T) == 4)
-    hipLaunchKernelGGL((prefill_kernel_f32<D>), dim3(nwg), dim3(kPThreads), 0, stream, pp);
-  else
-    hipLaunchKernelGGL((prefill_kernel<T, D>), dim3(nwg), dim3(kPThreads), 0, stream, pp);
+  const bool few = pp.Tq * pp.G <= kBM - 64;  // two waves or more without rows
+  if constexpr (sizeof(T) == 4) {
+    if (few)
+      hipLaunchKernelGGL((prefill_kernel_f32<D, true>), dim3(nwg), dim3(kPThreads), 0, stream, pp);
+    else
+      hipLaunchKernelGGL((prefill_kernel_f32<D, false>), dim3(nwg), dim3(kPThreads), 0, stream,
+                         pp);
+  } else {
+    if (few)
+      hipLaunchKernelGGL((prefill_kernel<T, D, true>), dim3(nwg), dim3(kPThreads), 0, stream, pp);
+    else
+      hipLaunchKernelGGL((prefill_kernel<T, D, false>), dim3(nwg), dim3(kPThreads), 0, stream, pp);
+  }
   const int st = launch_status("prefill_kernel");
   if (st || pp.splits == 1) return st;
   hipLaunchKernelGGL((prefill_merge_kernel<T, D>), dim3(pp.row_tiles * pp.Hkv * (D / 32)),
@@ -771,10 +803,14 @@ extern "C" int rlse_prefill_workspace_size(int num_tokens, int ctx_len, int num_
   if (num_tokens <= 0 || ctx_len < num_tokens || num_heads <= 0 || num_kv_heads <= 0 ||
       num_heads % num_kv_heads != 0 || (head_dim != 64 && head_dim != 128))
     return fail(RLSE_ERR_INVALID_VALUE, "prefill_workspace_size: bad shape");
-  PrefillPlan plan;
-  const int st = plan_prefill(num_tokens, ctx_len, num_heads, num_kv_heads, head_dim, &plan);
+  // The dtype is not known here: what either element size needs.
+  PrefillPlan p16, p32;
+  int st = plan_prefill(num_tokens, ctx_len, num_heads, num_kv_heads, head_dim, RLSE_DTYPE_BF16,
+                        &p16);
+  if (!st)
+    st = plan_prefill(num_tokens, ctx_len, num_heads, num_kv_heads, head_dim, RLSE_DTYPE_F32, &p32);
   if (st) return st;
-  *bytes = plan.ws_bytes;
+  *bytes = std::max(p16.ws_bytes, p32.ws_bytes);
   return RLSE_OK;
 }
 
@@ -791,7 +827,7 @@ extern "C" int rlse_prefill_attn(const void* q, const void* k_pool, const void* 
   if (!(scale > 0.f) || !isfinite(scale))
     return fail(RLSE_ERR_INVALID_VALUE, "prefill: scale must be finite and positive");
   PrefillPlan plan;
-  st = plan_prefill(num_tokens, ctx_len, num_heads, num_kv_heads, head_dim, &plan);
+  st = plan_prefill(num_tokens, ctx_len, num_heads, num_kv_heads, head_dim, dtype, &plan);
   if (st) return st;
   std::unique_lock<std::mutex> lock;
   if (plan.ws_bytes > 0) {
