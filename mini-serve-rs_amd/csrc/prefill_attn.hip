@@ -13,7 +13,8 @@
 // Tq*G rows (row = t*G + g). A workgroup of 8 waves takes 256 rows of one KV
 // head, each wave 32 of them, and streams that head's keys in tiles of 64:
 // the tile's K and V rows are staged in LDS once and shared by the 8
-// waves. When there are too few row tiles to fill the chip, the keys
+// waves (or, with two key groups, 128 rows over two tiles at a time, see
+// plan_prefill). When there are too few row tiles to fill the chip, the keys
 // are also split across workgroups: each stores its (m, l, acc) partial and
 // a second launch merges them with a log-sum-exp combine. Workgroups are mapped to
 // work so that consecutive work items -- the row tiles reading the same K/V
@@ -102,7 +103,9 @@ struct PrefillParams {
   void* out;           // [Tq][Hq][D]
   float* part;         // per-workgroup partial blocks (S > 1), see the kernel's tail
   int Tq, L, offset, Hq, Hkv, G, num_blocks, mbps;
-  int row_tiles, splits, split_keys;
+  int row_tiles;   // of a workgroup's rows (kBM, or kBM / 2 with two key groups)
+  int part_tiles;  // of kBM rows: the merge's tiles
+  int splits, split_keys;
   float c;  // scale * log2(e)
 };
 
@@ -110,7 +113,7 @@ struct PrefillParams {
 // float4 slots per thread of the workgroup.
 template <int D>
 __device__ __forceinline__ float4* part_block(const PrefillParams& p, int sp, int h, int rt) {
-  const size_t wgi = ((size_t)sp * p.Hkv + h) * p.row_tiles + rt;
+  const size_t wgi = ((size_t)sp * p.Hkv + h) * p.part_tiles + rt;
   return reinterpret_cast<float4*>(p.part) + wgi * (4 * (D / 32) + 1) * kPThreads;
 }
 
@@ -118,22 +121,30 @@ __device__ __forceinline__ float4* part_block(const PrefillParams& p, int sp, in
 // waves without any then only stage. (Left out otherwise: the branch around
 // the math costs the full kernel 3-9%; with 5 tokens of a group of 4 it takes
 // 8000 cached keys from 28.6 to 21.7 us.)
-template <typename T, int D, bool FEW>
+template <typename T, int D, int KG, bool FEW>
 __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) {
   constexpr int KB = D / 16;                  // 16-wide k-blocks of q.k
   constexpr int DB = D / 32;                  // 32-row blocks of O^T
   constexpr int CPR = D / 8;                  // 16-byte chunks per key row
-  constexpr int KPK = kBN * CPR;              // K packets per tile
+  constexpr int RG = kPWaves / KG;            // waves a key group has, 32 rows each
+  constexpr int BM = 32 * RG;                 // rows per workgroup
+  constexpr int STEP = kBN * KG;              // keys per step
+  constexpr int KPK = STEP * CPR;             // K packets per step
   constexpr int KPT = KPK / kPThreads;        // per thread
   static_assert(KPK % kPThreads == 0, "K tile must split evenly");
-  __shared__ __align__(16) uint16_t s_k[2][kBN][D + kPadK];  // K rows
-  __shared__ __align__(16) uint16_t s_v[2][kBN][D + kPadV];  // V rows
+  constexpr int KBYTES = 2 * STEP * (D + kPadK) * 2, VBYTES = 2 * STEP * (D + kPadV) * 2;
+  // The key groups' states meet in the same memory after the loop.
+  static_assert(KG == 1 || (4 * DB + 1) * RG * 64 * 16 <= KBYTES + VBYTES, "exchange fits");
+  __shared__ __align__(16) char s_kv[KBYTES + VBYTES];
+  auto& s_k = *reinterpret_cast<uint16_t(*)[2][STEP][D + kPadK]>(s_kv);           // K rows
+  auto& s_v = *reinterpret_cast<uint16_t(*)[2][STEP][D + kPadV]>(s_kv + KBYTES);  // V rows
   __shared__ int s_valid[2];                                 // page-valid bits of the tile
   __shared__ __align__(16) int s_pages[kMaxSplitPages];      // the split's page ids (-1: invalid)
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int half = lane >> 5, col = lane & 31;
+  const int rg = wave % RG, kg = wave / RG;  // row group, key group
 
   // XCD-aware work index: workgroup b runs on XCD b % 8; give each XCD a
   // contiguous run of work items.
@@ -146,16 +157,16 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
 
   const int G = p.G, Hq = p.Hq, Hkv = p.Hkv;
   const int rows = p.Tq * G;
-  const int myrow = rt * kBM + wave * 32 + col;
+  const int myrow = rt * BM + rg * 32 + col;
   const int row_c = myrow < rows ? myrow : rows - 1;
   const int t = row_c / G, g = row_c - t * G, qh = h * G + g;
-  const bool live = rt * kBM + wave * 32 < rows;  // the wave has rows (else it only stages)
+  const bool live = rt * BM + rg * 32 < rows;  // the wave has rows (else it only stages)
   const int kmax = p.offset + t;  // last key this query sees
   // Last key every query of this wave sees (its first row has the smallest t).
-  const int kmin_wave = p.offset + min(rt * kBM + wave * 32, rows - 1) / G;
+  const int kmin_wave = p.offset + min(rt * BM + rg * 32, rows - 1) / G;
 
   // Keys of this workgroup: up to the last query's diagonal, this split's share.
-  const int last_row = min(rows - 1, rt * kBM + kBM - 1);
+  const int last_row = min(rows - 1, rt * BM + BM - 1);
   const int wg_keys = min(p.L, p.offset + last_row / G + 1);
   const int k_begin = split * p.split_keys;
   const int k_end = min(wg_keys, k_begin + p.split_keys);
@@ -164,10 +175,10 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
   const T* __restrict__ kp = reinterpret_cast<const T*>(p.k_pool);
   const T* __restrict__ vp = reinterpret_cast<const T*>(p.v_pool);
 
-  // Page ids of this split's keys, staged once (whole 4-page tiles, indices
+  // Page ids of this split's keys, staged once (whole steps, indices
   // past the context clamped to its last page).
   {
-    const int npg = k_begin < k_end ? (((k_end - k_begin + 15) >> 4) + 3) & ~3 : 0;
+    const int npg = k_begin < k_end ? (((k_end - k_begin + 15) >> 4) + 4 * KG - 1) & -(4 * KG) : 0;
     const int plast = (p.L - 1) >> 4;
     for (int i = tid; i < npg; i += kPThreads) {
       const int pi = min((k_begin >> 4) + i, plast);
@@ -191,7 +202,7 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
       qreg[kb] = *reinterpret_cast<const uint4*>(qb + ((size_t)t * Hq + qh) * D + kb * 16 +
                                                  half * 8);
 
-   const int last_tile = k_begin + ((k_end - 1 - k_begin) / kBN) * kBN;
+    const int last_tile = k_begin + ((k_end - 1 - k_begin) / STEP) * STEP;
     static_assert(kBN == 64, "a tile spans 4 pages");
     // Packet u of this thread: key kk of the tile, 16-byte chunk dc of its
     // row. Its page, kk >> 4, is the same for the whole wave; its offset in
@@ -205,7 +216,7 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
       pg_of[u] = __builtin_amdgcn_readfirstlane(kk >> 4);
     }
     u32x4_t kst[KPT], vst[KPT];
-    int4 pid;  // page ids of the tile's 4 pages (-1: invalid), for the valid bits
+    int4 pid[KG];  // page ids of the tiles' 4 pages (-1: invalid), for the valid bits
     // Global loads of the tile at kt: raw buffer loads through a descriptor
     // of the packet's (page, head) tile, built in scalar registers. An
     // invalid page id gets a descriptor of zero records (zeros, no memory
@@ -213,7 +224,9 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
     // masked in the math.
     const size_t tile_elems = (size_t)16 * D;
     auto load_tile = [&](int kt) __attribute__((always_inline)) {
-      pid = *reinterpret_cast<const int4*>(&s_pages[(kt - k_begin) >> 4]);
+#pragma unroll
+      for (int t = 0; t < KG; ++t)
+        pid[t] = *reinterpret_cast<const int4*>(&s_pages[((kt - k_begin) >> 4) + 4 * t]);
 #pragma unroll
       for (int u = 0; u < KPT; ++u) {
         const int r = __builtin_amdgcn_readfirstlane(s_pages[((kt - k_begin) >> 4) + pg_of[u]]);
@@ -237,8 +250,12 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
         *reinterpret_cast<u32x4_t*>(&s_v[bf][kk][dc * 8]) = vst[u];
       }
       if (tid == 0) {
-        s_valid[bf] = (pid.x >= 0 ? 1 : 0) | (pid.y >= 0 ? 2 : 0) | (pid.z >= 0 ? 4 : 0) |
-                      (pid.w >= 0 ? 8 : 0);
+        int bits = 0;
+#pragma unroll
+        for (int t = 0; t < KG; ++t)
+          bits |= ((pid[t].x >= 0 ? 1 : 0) | (pid[t].y >= 0 ? 2 : 0) | (pid[t].z >= 0 ? 4 : 0) |
+                   (pid[t].w >= 0 ? 8 : 0)) << (4 * t);
+        s_valid[bf] = bits;
       }
     };
     // V^T operand reads: lane = (group g of 16, j = key row in the group's
@@ -251,10 +268,11 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
     store_tile(0);
     __syncthreads();
     int bf = 0;
-    for (int kt = k_begin;; kt += kBN) {
-      const bool more = kt < last_tile;
-      load_tile(more ? kt + kBN : kt);  // in flight during this tile's math
-      const int vbits = s_valid[bf];
+    for (int k0 = k_begin;; k0 += STEP) {
+      const bool more = k0 < last_tile;
+      load_tile(more ? k0 + STEP : k0);  // in flight during this step's math
+      const int kt = k0 + kBN * kg;      // this wave's tile (past the end: all masked)
+      const int vbits = (s_valid[bf] >> (4 * kg)) & 15;
 
       if (!FEW || live) {
       // S^T for the two 32-key halves of the tile.
@@ -270,7 +288,7 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
 #pragma unroll
         for (int sb = 0; sb < 2; ++sb) {
           const uint4 a =
-              *reinterpret_cast<const uint4*>(&s_k[bf][sb * 32 + col][kb * 16 + half * 8]);
+              *reinterpret_cast<const uint4*>(&s_k[bf][kBN * kg + sb * 32 + col][kb * 16 + half * 8]);
           s[sb] = Mfma<T>::mma(a, qreg[kb], s[sb]);
         }
       // Mask (causal, past the split's end, invalid pages) only on tiles that
@@ -330,7 +348,7 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
       for (int kq = 0; kq < 4; ++kq)
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-          const uint16_t* v0 = &s_v[bf][kq * 16 + tr_row][db * 32 + tr_col];
+          const uint16_t* v0 = &s_v[bf][kBN * kg + kq * 16 + tr_row][db * 32 + tr_col];
           const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)v0);
           const i16x4_t hi =
               __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(v0 + 8 * (D + kPadV)));
@@ -344,6 +362,41 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
       __syncthreads();
       bf ^= 1;
     }
+  }
+
+  if constexpr (KG > 1) {
+    // The second key group hands its state to the first, which combines the
+    // two (log-sum-exp) and finishes the rows.
+    static_assert(KG == 2, "two key groups");
+    float4* ex = reinterpret_cast<float4*>(s_kv) + (rg * 64 + lane);
+    __syncthreads();
+    if (kg == 1) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4)
+          ex[(db * 4 + i4) * RG * 64] =
+              make_float4(o[db][i4 * 4], o[db][i4 * 4 + 1], o[db][i4 * 4 + 2], o[db][i4 * 4 + 3]);
+      ex[4 * DB * RG * 64] = make_float4(m, lsum, 0.f, 0.f);
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    const float4 ml = ex[4 * DB * RG * 64];
+    const float mn = fmaxf(m, ml.x);
+    const float sa = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+    const float sb = mn == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - mn);
+    m = mn;
+    lsum = lsum * sa + ml.y * sb;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) {
+        const float4 x = ex[(db * 4 + i4) * RG * 64];
+        o[db][i4 * 4] = o[db][i4 * 4] * sa + x.x * sb;
+        o[db][i4 * 4 + 1] = o[db][i4 * 4 + 1] * sa + x.y * sb;
+        o[db][i4 * 4 + 2] = o[db][i4 * 4 + 2] * sa + x.z * sb;
+        o[db][i4 * 4 + 3] = o[db][i4 * 4 + 3] * sa + x.w * sb;
+      }
   }
 
   // Lane holds O^T rows d = 32*db + 8*(i/4) + 4*half + i%4 of its query.
@@ -370,7 +423,8 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
   // (m, l) -- so every store covers 1 KB of consecutive bytes. The merge
   // launch reads them back with the same thread-to-row map.
   if (!live) return;  // the merge reads no row of this wave
-  float4* blk = part_block<D>(p, split, h, rt) + tid;
+  // (KG row tiles share a block, as the merge's 256-row tiles hold them.)
+  float4* blk = part_block<D>(p, split, h, rt / KG) + (rt % KG) * RG * 64 + rg * 64 + lane;
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -638,7 +692,7 @@ __global__ __launch_bounds__(kPThreads) void prefill_merge_kernel(PrefillParams 
   const int wave = tid >> 6, lane = tid & 63, half = lane >> 5, col = lane & 31;
   const int q = blockIdx.x % DB;
   const int tile = blockIdx.x / DB;
-  const int rt = tile % p.row_tiles, h = tile / p.row_tiles;
+  const int rt = tile % p.part_tiles, h = tile / p.part_tiles;
   const int G = p.G, Hq = p.Hq;
   const int rows = p.Tq * G;
   const int myrow = rt * kBM + wave * 32 + col;
@@ -700,65 +754,93 @@ __global__ __launch_bounds__(kPThreads) void prefill_merge_kernel(PrefillParams 
 
 // Workspace (key splits only): the partial blocks of every workgroup.
 struct PrefillPlan {
-  int row_tiles, splits, split_keys;
+  int row_tiles, part_tiles, key_groups, splits, split_keys;
   size_t ws_bytes;
 };
 
-// Splits of the keys: the count with the least estimated time, in us,
-//   rounds of workgroups over the compute units x tiles per split x t
+// Key groups of a workgroup and splits of the keys: the pair with the least
+// estimated time, in us,
+//   rounds of workgroups over the compute units x steps per split x t
+//   + (two key groups) 15% a step and the exchange
 //   + (more than one split) the merge launch, a round trip per kMergeBatch
 //     splits and the partial blocks written and read back.
 // t is a tile's time in a workgroup, measured on one split of long contexts.
-// Measured against one workgroup per compute unit with at least 512 keys
-// each: f32, 16/8 heads of 128, 333 tokens after 1030: 8 splits for 3, 135 ->
-// 68 us; 20 tokens after 1030: 17 for 3, 97 -> 32 us; bf16, 14/2 heads of 64,
-// 2000 tokens: 2 for 3 (one round for two), 36 -> 33 us.
+// Two key groups (16-bit, d = 128; half the rows a workgroup, two tiles of
+// keys at once, the halves combined in LDS) fill the chip without partial
+// blocks or a merge where rows are few: bf16, 16/8 heads, 1000 tokens 31.1 ->
+// 24.9 us, 400 tokens 18.8 -> 14.1; with rows for every compute unit they lose
+// (32/8 heads, 512 tokens after 8192: 95.2 against 99.0), and so they do over
+// one or two tiles a split (one token after 100: 7.0 against 7.6).
+// Splits, measured against one workgroup per compute unit with at least 512
+// keys each: f32, 16/8 heads of 128, 333 tokens after 1030: 8 splits for 3,
+// 135 -> 68 us; 20 tokens after 1030: 17 for 3, 97 -> 22 us; bf16, 14/2 heads of
+// 64, 2000 tokens: 2 for 3 (one round for two), 36 -> 33 us.
 int plan_prefill(int Tq, int ctx_len, int Hq, int Hkv, int D, int dtype, PrefillPlan* plan) {
   int cus = 0;
   const int st = device_cu_count(&cus);
   if (st) return st;
   const int G = Hq / Hkv;
-  plan->row_tiles = (Tq * G + kBM - 1) / kBM;
-  const long long base = (long long)plan->row_tiles * Hkv;
+  const int rows = Tq * G;
+  plan->part_tiles = (rows + kBM - 1) / kBM;
   const size_t block = (size_t)(4 * (D / 32) + 1) * kPThreads * 4 * sizeof(float);
   const double tile_us = dtype == RLSE_DTYPE_F32 ? (D == 128 ? 14.7 : 7.7) : (D == 128 ? 1.9 : 1.2);
   const int tiles = (ctx_len + kBN - 1) / kBN;
   const int most = kMaxSplitPages * 16 / kBN;  // a split's page ids must fit the LDS stage
   const int limit = std::min(tiles, std::max(kMaxSplits, (tiles + most - 1) / most));
-  int best = 0, best_per = 0;
   double best_us = 0.;
-  for (int want = 1; want <= limit; ++want) {
-    const int per = (tiles + want - 1) / want, s = (tiles + per - 1) / per;
-    if (s != want || per > most) continue;  // (fewer splits gave the same shares)
-    double us = (double)((base * s + cus - 1) / cus) * per * tile_us;
-    if (s > 1) us += 3. + 1.5 * ((s + kMergeBatch - 1) / kMergeBatch) + 2. * base * s * block / 4e6;
-    if (best == 0 || us < best_us) best = s, best_per = per, best_us = us;
+  plan->splits = 0;
+  for (int kg = 1; kg <= (dtype != RLSE_DTYPE_F32 && D == 128 ? 2 : 1); ++kg) {
+    const int row_tiles = (rows + kBM / kg - 1) / (kBM / kg);
+    const long long base = (long long)row_tiles * Hkv;
+    for (int want = 1; want <= limit; ++want) {
+      const int per = (tiles + want - 1) / want, s = (tiles + per - 1) / per;
+      if (s != want || per > most) continue;  // (fewer splits gave the same shares)
+      if (kg > 1 && per <= 2) continue;
+      const int steps = (per + kg - 1) / kg;
+      double us = (double)((base * s + cus - 1) / cus) * steps * tile_us;
+      if (kg > 1) us = us * 1.15 + 1.2;
+      if (s > 1)
+        us += 3. + 1.5 * ((s + kMergeBatch - 1) / kMergeBatch) + 2. * base * s * block / kg / 4e6;
+      if (plan->splits == 0 || us < best_us) {
+        best_us = us;
+        plan->row_tiles = row_tiles;
+        plan->key_groups = kg;
+        plan->splits = s;
+        plan->split_keys = per * kBN;
+      }
+    }
   }
-  plan->splits = best;
-  plan->split_keys = best_per * kBN;
-  plan->ws_bytes = best > 1 ? (size_t)best * base * block : 0;
+  plan->ws_bytes = plan->splits > 1 ? (size_t)plan->splits * plan->part_tiles * Hkv * block : 0;
   return RLSE_OK;
 }
 
 template <typename T, int D>
-int launch_prefill(PrefillParams& pp, hipStream_t stream) {
+int launch_prefill(PrefillParams& pp, int key_groups, hipStream_t stream) {
   const int nwg = pp.row_tiles * pp.Hkv * pp.splits;
-  const bool few = pp.Tq * pp.G <= kBM - 64;  // two waves or more without rows
+  const int bm = kBM / key_groups;
+  const bool few = pp.Tq * pp.G <= bm - 64;  // two waves or more without rows
+  const dim3 grid(nwg), block(kPThreads);
   if constexpr (sizeof(T) == 4) {
     if (few)
-      hipLaunchKernelGGL((prefill_kernel_f32<D, true>), dim3(nwg), dim3(kPThreads), 0, stream, pp);
+      hipLaunchKernelGGL((prefill_kernel_f32<D, true>), grid, block, 0, stream, pp);
     else
-      hipLaunchKernelGGL((prefill_kernel_f32<D, false>), dim3(nwg), dim3(kPThreads), 0, stream,
-                         pp);
+      hipLaunchKernelGGL((prefill_kernel_f32<D, false>), grid, block, 0, stream, pp);
   } else {
-    if (few)
-      hipLaunchKernelGGL((prefill_kernel<T, D, true>), dim3(nwg), dim3(kPThreads), 0, stream, pp);
+    auto run = [&](auto kg) {
+      constexpr int KG = decltype(kg)::value;
+      if (few)
+        hipLaunchKernelGGL((prefill_kernel<T, D, KG, true>), grid, block, 0, stream, pp);
+      else
+        hipLaunchKernelGGL((prefill_kernel<T, D, KG, false>), grid, block, 0, stream, pp);
+    };
+    if (D == 128 && key_groups == 2)
+      run(std::integral_constant<int, D == 128 ? 2 : 1>{});
     else
-      hipLaunchKernelGGL((prefill_kernel<T, D, false>), dim3(nwg), dim3(kPThreads), 0, stream, pp);
+      run(std::integral_constant<int, 1>{});
   }
   const int st = launch_status("prefill_kernel");
   if (st || pp.splits == 1) return st;
-  hipLaunchKernelGGL((prefill_merge_kernel<T, D>), dim3(pp.row_tiles * pp.Hkv * (D / 32)),
+  hipLaunchKernelGGL((prefill_merge_kernel<T, D>), dim3(pp.part_tiles * pp.Hkv * (D / 32)),
                      dim3(kPThreads), 0, stream, pp);
   return launch_status("prefill_merge_kernel");
 }
@@ -867,14 +949,15 @@ extern "C" int rlse_prefill_attn(const void* q, const void* k_pool, const void* 
   pp.num_blocks = num_blocks;
   pp.mbps = max_blocks;
   pp.row_tiles = plan.row_tiles;
+  pp.part_tiles = plan.part_tiles;
   pp.splits = plan.splits;
   pp.split_keys = plan.split_keys;
   pp.c = scale * 1.4426950408889634f;
   const hipStream_t s = as_stream(stream);
   if (dtype == RLSE_DTYPE_BF16)
-    return head_dim == 128 ? launch_prefill<bf16, 128>(pp, s) : launch_prefill<bf16, 64>(pp, s);
+    return head_dim == 128 ? launch_prefill<bf16, 128>(pp, plan.key_groups, s) : launch_prefill<bf16, 64>(pp, plan.key_groups, s);
   if (dtype == RLSE_DTYPE_F32)
-    return head_dim == 128 ? launch_prefill<float, 128>(pp, s)
-                           : launch_prefill<float, 64>(pp, s);
-  return head_dim == 128 ? launch_prefill<f16, 128>(pp, s) : launch_prefill<f16, 64>(pp, s);
+    return head_dim == 128 ? launch_prefill<float, 128>(pp, plan.key_groups, s)
+                           : launch_prefill<float, 64>(pp, plan.key_groups, s);
+  return head_dim == 128 ? launch_prefill<f16, 128>(pp, plan.key_groups, s) : launch_prefill<f16, 64>(pp, plan.key_groups, s);
 }

@@ -188,3 +188,27 @@ def test_prefill_single_token_equals_decode(kv, dtype):
     mx, rel = err_report(as_f32(got, dtype), as_f32(dec, dtype))
     print(f"[prefill(1) vs decode] max_abs={mx:.3e} rel={rel:.3e}")
     assert mx <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("hq,hkv,d,tq,offset", [
+    (16, 8, 128, 32, 200),   # 64 rows: the last chunk whose spare waves only stage (2 key groups)
+    (16, 8, 128, 33, 200),   # 66 rows
+    (16, 8, 128, 65, 130),   # 130 rows: two half tiles, four tiles of keys
+    (4, 1, 128, 3, 2000),    # many splits, an odd number of tiles in some
+    (4, 1, 128, 150, 4100),  # 600 rows after a long context: splits and two key groups
+    (14, 2, 64, 27, 300),    # 189 rows of 256: spare waves, one key group
+    (14, 2, 64, 28, 301)])   # 196 rows
+def test_prefill_row_and_key_groups_match_oracle(kv, dtype, hq, hkv, d, tq, offset):
+    """Chunks around the edges of the row tiles, the key groups and the
+    splits, one page id outside the pool never read (its keys invisible to no
+    query: past the context)."""
+    rng = np.random.default_rng(tq * 7 + offset)
+    q, kp, vp, table, L = make_case(rng, hq, hkv, d, tq, offset, dtype)
+    scale = 1.0 / np.sqrt(d)
+    table = np.concatenate([table, np.array([kp.shape[0] + 5], np.int32)])
+    got = as_f32(run_prefill(kv, q, kp, vp, table, L, hq, hkv, d, dtype, scale), dtype)
+    want = oracle_prefill(q, kp, vp, table, L, hq, hkv, d, dtype, scale)
+    mx, rel = err_report(got, want)
+    print(f"[prefill groups {hq}/{hkv}/{d} {tq}+{offset}] {dtype} max_abs={mx:.3e} rel={rel:.3e}")
+    assert np.isfinite(got).all() and mx <= TOL[dtype]
