@@ -560,6 +560,21 @@ int rlse_gate_up_silu(const void* x, const void* w_gate_up, void* act, int rows,
                       int inter, int dtype, void* workspace, size_t workspace_bytes,
                       rlse_stream_t stream);
 
+/* input_layernorm + q/k/v_proj and post_attention_layernorm + the MLP front
+ * of the decode step (qwen2.rs:668-679, 750-753): rlse_add_rmsnorm(NULL,
+ * residual, norm_weight, h) followed by rlse_qkv_proj / rlse_gate_up_silu on
+ * h, in one launch for a decode batch of up to 16 rows whose shape allows it.
+ * residual is row-major and only read; h (whole 16-row tiles) is scratch,
+ * its contents afterwards unspecified. */
+int rlse_norm_qkv_proj(const void* residual, const void* norm_weight, float eps, void* h,
+                       const void* w_qkv, const void* b_qkv, void* q, void* k, void* v, int rows,
+                       int hidden, int q_features, int kv_features, int dtype, void* workspace,
+                       size_t workspace_bytes, rlse_stream_t stream);
+int rlse_norm_gate_up_silu(const void* residual, const void* norm_weight, float eps, void* h,
+                           const void* w_gate_up, void* act, int rows, int hidden, int inter,
+                           int dtype, void* workspace, size_t workspace_bytes,
+                           rlse_stream_t stream);
+
 /* ------------------------------------------------------------------ */
 /* Host block manager: the physical successor of KVCache               */
 /* (src/cache/kv_cache.rs:15-145) with per-block refcounts for prefix  */

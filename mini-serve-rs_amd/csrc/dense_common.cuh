@@ -69,6 +69,9 @@ struct DenseParams {
   int packed;        // w in the tile order rlse_dense_pack writes
   int xpacked;       // x in the packed row order (RLSE_PACKED_ROWS)
   int opacked;       // kEpiSiluMul: act in the packed row order (RLSE_PACKED_OUT)
+  const void* norm_w;  // RMSNorm weight [K]: x is the raw residual (null: x as it is)
+  void* norm_h;        // [whole 16-row tiles][K], where the norm is a launch of its own
+  float eps, inv_k;
 };
 
 template <typename T>

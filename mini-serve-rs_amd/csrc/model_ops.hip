@@ -299,7 +299,13 @@ constexpr int kDenseHeaderWords = 64;
 // order the split grid's merge adds its records (the waves of a slice in
 // order, then the slices in order), so the results are the split grid's to
 // the bit. No records, no launch counters, no second round trip to memory.
-template <typename T, int RT, int FT, int EPI, int KV = 1>
+//
+// NU > 0: x is the raw residual stream (row-major) and its RMSNorm runs here,
+// in place of a launch of norm_rows_kernel before: a wave holds all its k
+// steps (at most NU) of x and of the weights, the waves' sums of squares meet
+// in LDS while the weights are on their way, and each wave normalises its
+// own operands in registers, rounded as norm_rows_kernel rounds them.
+template <typename T, int RT, int FT, int EPI, int KV = 1, int NU = 0>
 __global__ __launch_bounds__(64 * kDenseWaves * KV) void dense_rows_kernel(DenseParams p) {
   constexpr int WV = kDenseWaves * KV;  // waves per workgroup
   if constexpr (KV > 1 && RT == 1 && (EPI == kEpiResidual || EPI == kEpiQkv)) {
@@ -413,7 +419,82 @@ __global__ __launch_bounds__(64 * kDenseWaves * KV) void dense_rows_kernel(Dense
   const int slice_end = (sl + 1) * S / NS;
   const int s_begin = sl * S / NS + ws * p.steps;
   const int s_end = min(slice_end, s_begin + p.steps);
-  for (int s = s_begin; s < s_end; s += U) {
+  if constexpr (NU > 0) {
+    // Every load is unconditional (steps past the wave's last re-read it and
+    // are not used), so the waits below count loads and x is worked on while
+    // the weights arrive.
+    __shared__ float s_ss[WV][RT][16];
+    u32x4_t a[NU][FT], b[NU][RT], nw[NU];
+    const int last = s_end > s_begin ? s_end - 1 : S - 1;
+#pragma unroll
+    for (int j = 0; j < NU; ++j) {
+      const int s = min(s_begin + j, last);
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+        b[j][t] = *reinterpret_cast<const u32x4_t*>(xr[t] + (size_t)xstep * s);
+    }
+#pragma unroll
+    for (int j = 0; j < NU; ++j)
+      nw[j] = *reinterpret_cast<const u32x4_t*>((const T*)p.norm_w + SE * min(s_begin + j, last) +
+                                                (SE / 4) * g);
+#pragma unroll
+    for (int j = 0; j < NU; ++j)
+#pragma unroll
+      for (int f = 0; f < FT; ++f)
+        a[j][f] = *reinterpret_cast<const u32x4_t*>(wr[f] +
+                                                    (size_t)wstep * min(s_begin + j, last));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < NU; ++j) {
+        float h[8], part = 0.f;
+        Packet<T>::unpack(__builtin_bit_cast(uint4, b[j][t]), h);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) part = fmaf(h[e], h[e], part);
+        ss += s_begin + j < s_end ? part : 0.f;
+      }
+      ss += __shfl_xor(ss, 16, 64);
+      ss += __shfl_xor(ss, 32, 64);
+      if (g == 0) s_ss[wave][t][fi] = ss;
+    }
+    // A barrier for LDS alone: the weights stay in flight.
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      float ss = 0.f;
+#pragma unroll
+      for (int w = 0; w < WV; ++w) ss += s_ss[w][t][fi];
+      // h / norm as the rounded reciprocal's product and one correction of its
+      // remainder, which rounds as the division does; an overflowed sum gives
+      // 0, as h / inf.
+      float norm = sqrtf(ss * p.inv_k + p.eps);
+      const float y = 1.f / norm;
+      norm = y == 0.f ? 0.f : norm;
+#pragma unroll
+      for (int j = 0; j < NU; ++j) {
+        float h[8], w[8], o[8];
+        Packet<T>::unpack(__builtin_bit_cast(uint4, b[j][t]), h);
+        Packet<T>::unpack(__builtin_bit_cast(uint4, nw[j]), w);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float q = h[e] * y;
+          o[e] = round_cvt<T>(fmaf(fmaf(-q, norm, h[e]), y, q)) * w[e];
+        }
+        b[j][t] = __builtin_bit_cast(u32x4_t, cvt_packet<T>(o));
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NU; ++j)
+      if (s_begin + j < s_end) {
+#pragma unroll
+        for (int f = 0; f < FT; ++f)
+#pragma unroll
+          for (int t = 0; t < RT; ++t) acc[f][t] = Mma16<T>::run(a[j][f], b[j][t], acc[f][t]);
+      }
+  }
+  for (int s = s_begin; NU == 0 && s < s_end; s += U) {
     u32x4_t a[U][FT], b[U][RT];
 #pragma unroll
     for (int j = 0; j < U; ++j) {
@@ -596,6 +677,29 @@ int by_dtype(int dtype, F&& f) {
   return fail(RLSE_ERR_INVALID_VALUE, "bad dtype %d", dtype);
 }
 
+// [residual add and] RMSNorm; chunked: rows of whole 16-byte chunks, at most
+// kNormThreads * kNormChunks of them, in 16-byte aligned buffers (packed_out
+// only then).
+template <typename T>
+int launch_norm(const T* x, T* residual, const T* w, T* out, int rows, int n, float eps,
+                bool chunked, bool packed_out, hipStream_t s) {
+  const float inv_n = (float)(1.0 / (double)n);
+  auto run = [&](auto add) {
+    constexpr bool ADD = decltype(add)::value;
+    if (chunked)
+      hipLaunchKernelGGL((norm_rows_kernel<T, ADD>), dim3(rows), dim3(kNormThreads), 0, s, x,
+                         residual, w, out, n, inv_n, eps, (int)packed_out);
+    else
+      hipLaunchKernelGGL((norm_rows_any_kernel<T, ADD>), dim3((rows + 3) / 4), dim3(256), 0, s, x,
+                         residual, w, out, rows, n, inv_n, eps);
+  };
+  if (x)
+    run(std::true_type{});
+  else
+    run(std::false_type{});
+  return launch_status("add_rmsnorm");
+}
+
 // One rocBLAS handle per device, created on first use.
 std::mutex g_blas_mu;
 rocblas_handle g_blas[64] = {nullptr};
@@ -643,6 +747,21 @@ bool dense_long_k(int groups, int rows, int K) {
   return K >= 96 * 32 && groups * ((rows + 15) / 16) <= 512;
 }
 
+// Whether the norm before a product runs in its launch: every wave must hold
+// its k steps of x (8, or 2 in a 16-wave workgroup) and every workgroup all of
+// K, for at most kDenseNormRows rows. A launch costs about 4 us between two
+// others, the norm of one row tile about 1 us of VALU time in each workgroup:
+// whole steps, Qwen2.5-0.5B, one user: 1022 -> 968 us; with two row tiles
+// (Qwen3-0.6B, 32 users) the step took 1849 against 1780 us.
+constexpr int kDenseNormRows = 16;
+template <int EPI>
+bool dense_norm_fits(const DenseParams& p, int ft, int ks, int kv_inner) {
+  if ((EPI != kEpiQkv && EPI != kEpiSiluMul) || p.rows > kDenseNormRows || ft != 1) return false;
+  const int steps = p.K / 32;
+  if (kv_inner > 1) return EPI == kEpiQkv && kv_inner == 4 && ((steps + 3) / 4 + kDenseWaves - 1) / kDenseWaves <= 2;
+  return ks == 1 && (steps + kDenseWaves - 1) / kDenseWaves <= 8;
+}
+
 // Launches a product: dense_rows_kernel for a decode batch, the tiled kernel
 // for more rows. Shapes were checked by the caller:
 // K % 32 == 0, 16-feature tiles that never straddle an output, 16-byte
@@ -668,6 +787,18 @@ int launch_dense(DenseParams p, size_t ws_words, hipStream_t s) {
        (p.rows <= 32 || EPI == kEpiResidual || EPI == kEpiQkv))
           ? std::min(ks, kDenseMaxInner)
           : 1;
+  const bool norm = p.norm_w != nullptr;
+  if (norm && !dense_norm_fits<EPI>(p, ft, ks, kv_inner)) {
+    // The norm as a launch of its own, its rows packed where they can be.
+    const bool chunked = p.K <= kNormThreads * kNormChunks * 8;
+    const int rc = launch_norm<T>(nullptr, (T*)const_cast<void*>(p.x), (const T*)p.norm_w,
+                                  (T*)p.norm_h, p.rows, p.K, p.eps, chunked, chunked, s);
+    if (rc) return rc;
+    p.x = p.norm_h;
+    p.xpacked = chunked;
+    p.norm_w = nullptr;
+    return launch_dense<T, EPI>(p, ws_words, s);
+  }
   if constexpr (EPI != kEpiStore) {  // plain stores come 64 rows at a time
     if (p.rows > kDenseMaxRows && !(kv_inner > 1 && dense_long_k(groups, p.rows, p.K)))
       return launch_dense_tile(EPI, std::is_same<T, bf16>::value ? RLSE_DTYPE_BF16 : RLSE_DTYPE_F16,
@@ -688,6 +819,25 @@ int launch_dense(DenseParams p, size_t ws_words, hipStream_t s) {
   const dim3 grid(groups * p.ksplit);
   auto run = [&](auto rt_c) {
     constexpr int RT = decltype(rt_c)::value;
+    if constexpr (sizeof(T) == 2 && RT == 1 && (EPI == kEpiQkv || EPI == kEpiSiluMul)) {
+      if (norm) {
+        if constexpr (EPI == kEpiQkv) {
+          if (kv_inner > 1) {
+            hipLaunchKernelGGL((dense_rows_kernel<T, 1, 1, EPI, 4, 2>), dim3(grid.x, rt),
+                               dim3(64 * kDenseWaves * 4), 0, s, p);
+            return;
+          }
+        }
+        // Two tiles a workgroup where 256 such groups are left: each norms
+        // the rows for itself (Qwen2.5-0.5B, one user, whole step 979 -> 968 us).
+        if (tiles % 2 == 0 && tiles / 2 >= 256)
+          hipLaunchKernelGGL((dense_rows_kernel<T, RT, 2, EPI, 1, 8>), dim3(tiles / 2), block, 0,
+                             s, p);
+        else
+          hipLaunchKernelGGL((dense_rows_kernel<T, RT, 1, EPI, 1, 8>), grid, block, 0, s, p);
+        return;
+      }
+    }
     if constexpr ((RT <= 2 || EPI == kEpiResidual || EPI == kEpiQkv) && EPI != kEpiSiluMul) {
       if (kv_inner > 1) {
         // A residual or q/k/v projection's row tiles go to separate
@@ -794,6 +944,31 @@ int dense_workspace(const char* what, DenseParams& p, void* workspace, size_t wo
   return RLSE_OK;
 }
 
+// The RMSNorm of a norm + projection call: x is then the raw residual.
+struct Norm {
+  bool on = false;
+  const void* weight = nullptr;
+  void* h = nullptr;  // whole 16-row tiles, for shapes that norm in a launch of their own
+  float eps = 0.f;
+  void set(DenseParams& p) const {
+    if (!on) return;
+    p.norm_w = weight;
+    p.norm_h = h;
+    p.eps = eps;
+    p.inv_k = (float)(1.0 / (double)p.K);
+  }
+};
+
+int check_norm(const char* what, const Norm& norm, const DenseParams& flags) {
+  if (!norm.on) return RLSE_OK;
+  if (!(norm.eps >= 0.f)) return fail(RLSE_ERR_INVALID_VALUE, "%s: eps must be >= 0", what);
+  if (!norm.weight || !norm.h) return fail(RLSE_ERR_INVALID_VALUE, "%s: null pointer", what);
+  if (flags.xpacked || !aligned(norm.weight, 16) || !aligned(norm.h, 16))
+    return fail(RLSE_ERR_INVALID_VALUE,
+                "%s: a row-major residual, norm weight and h 16-byte aligned", what);
+  return RLSE_OK;
+}
+
 // Weights in the tile order of dense_rows_kernel: one 16-byte packet per
 // thread, packet i = ((tile * K/32 + s) * 64 + lane) holding row
 // row(tile, lane % 16), elements 32s + 8(lane / 16) .. +8. Rows of a tile are
@@ -857,7 +1032,6 @@ extern "C" int rlse_add_rmsnorm(const void* x, void* residual, const void* weigh
   if (rows == 0) return RLSE_OK;
   if (!residual || !weight || !out)
     return fail(RLSE_ERR_INVALID_VALUE, "add_rmsnorm: null pointer");
-  const float inv_n = (float)(1.0 / (double)n);
   hipStream_t s = as_stream(stream);
   const bool chunked = (n * es) % 16 == 0 && n * es / 16 <= (size_t)kNormThreads * kNormChunks &&
                        aligned(residual, 16) && aligned(weight, 16) && aligned(out, 16) &&
@@ -868,23 +1042,8 @@ extern "C" int rlse_add_rmsnorm(const void* x, void* residual, const void* weigh
                 "16-byte aligned buffers", kNormThreads * kNormChunks * 8);
   return by_dtype(dtype, [&](auto t) {
     using T = decltype(t);
-    const T* xp = (const T*)x;
-    T* rp = (T*)residual;
-    if (chunked) {
-      if (x)
-        hipLaunchKernelGGL((norm_rows_kernel<T, true>), dim3(rows), dim3(kNormThreads), 0, s,
-                           xp, rp, (const T*)weight, (T*)out, n, inv_n, eps, (int)packed_out);
-      else
-        hipLaunchKernelGGL((norm_rows_kernel<T, false>), dim3(rows), dim3(kNormThreads), 0, s,
-                           xp, rp, (const T*)weight, (T*)out, n, inv_n, eps, (int)packed_out);
-    } else if (x) {
-      hipLaunchKernelGGL((norm_rows_any_kernel<T, true>), dim3((rows + 3) / 4), dim3(256), 0, s,
-                         xp, rp, (const T*)weight, (T*)out, rows, n, inv_n, eps);
-    } else {
-      hipLaunchKernelGGL((norm_rows_any_kernel<T, false>), dim3((rows + 3) / 4), dim3(256), 0,
-                         s, xp, rp, (const T*)weight, (T*)out, rows, n, inv_n, eps);
-    }
-    return launch_status("add_rmsnorm");
+    return launch_norm<T>((const T*)x, (T*)residual, (const T*)weight, (T*)out, rows, n, eps,
+                          chunked, packed_out, s);
   });
 }
 
@@ -1046,21 +1205,23 @@ extern "C" int rlse_dense_workspace_size(int rows, int out_features, int in_feat
   return RLSE_OK;
 }
 
-extern "C" int rlse_qkv_proj(const void* x, const void* w_qkv, const void* b_qkv, void* q,
-                             void* k, void* v, int rows, int hidden, int q_features,
-                             int kv_features, int dtype, void* workspace, size_t workspace_bytes,
-                             rlse_stream_t stream) {
+static int qkv_proj(const char* what, const Norm& norm, const void* x, const void* w_qkv,
+                    const void* b_qkv, void* q, void* k, void* v, int rows, int hidden,
+                    int q_features, int kv_features, int dtype, void* workspace,
+                    size_t workspace_bytes, rlse_stream_t stream) {
   DenseParams flags{};
   take_packed(dtype, flags);
   const void* outs[3] = {q, k, v};
-  int rc = check_dense("qkv_proj", dtype, rows, hidden, x, w_qkv, outs, 3);
+  int rc = check_dense(what, dtype, rows, hidden, x, w_qkv, outs, 3);
   if (rc || rows == 0) return rc;
+  rc = check_norm(what, norm, flags);
+  if (rc) return rc;
   if (q_features <= 0 || kv_features <= 0 || q_features % 16 || kv_features % 16)
     return fail(RLSE_ERR_INVALID_VALUE,
-                "qkv_proj: q_features %d and kv_features %d must be positive multiples of 16",
-                q_features, kv_features);
+                "%s: q_features %d and kv_features %d must be positive multiples of 16",
+                what, q_features, kv_features);
   if (b_qkv && !aligned(b_qkv, 8))
-    return fail(RLSE_ERR_INVALID_VALUE, "qkv_proj: bias must be 8-byte aligned");
+    return fail(RLSE_ERR_INVALID_VALUE, "%s: bias must be 8-byte aligned", what);
   DenseParams p{};
   p.x = x;
   p.w = w_qkv;
@@ -1075,10 +1236,29 @@ extern "C" int rlse_qkv_proj(const void* x, const void* w_qkv, const void* b_qkv
   p.N = q_features + 2 * kv_features;
   p.packed = flags.packed;
   p.xpacked = flags.xpacked;
+  norm.set(p);
   size_t words = 0;
-  rc = dense_workspace("qkv_proj", p, workspace, workspace_bytes, &words);
+  rc = dense_workspace(what, p, workspace, workspace_bytes, &words);
   if (rc) return rc;
   return dense_by_dtype<kEpiQkv>(dtype, p, words, as_stream(stream));
+}
+
+extern "C" int rlse_qkv_proj(const void* x, const void* w_qkv, const void* b_qkv, void* q,
+                             void* k, void* v, int rows, int hidden, int q_features,
+                             int kv_features, int dtype, void* workspace, size_t workspace_bytes,
+                             rlse_stream_t stream) {
+  return qkv_proj("qkv_proj", Norm{}, x, w_qkv, b_qkv, q, k, v, rows, hidden, q_features,
+                  kv_features, dtype, workspace, workspace_bytes, stream);
+}
+
+extern "C" int rlse_norm_qkv_proj(const void* residual, const void* norm_weight, float eps,
+                                  void* h, const void* w_qkv, const void* b_qkv, void* q, void* k,
+                                  void* v, int rows, int hidden, int q_features, int kv_features,
+                                  int dtype, void* workspace, size_t workspace_bytes,
+                                  rlse_stream_t stream) {
+  return qkv_proj("norm_qkv_proj", Norm{true, norm_weight, h, eps}, residual, w_qkv, b_qkv, q, k,
+                  v, rows, hidden, q_features, kv_features, dtype, workspace, workspace_bytes,
+                  stream);
 }
 
 extern "C" int rlse_linear_residual(const void* x, const void* weight, void* residual, int rows,
@@ -1109,20 +1289,22 @@ extern "C" int rlse_linear_residual(const void* x, const void* weight, void* res
   return dense_by_dtype<kEpiResidual>(dtype, p, words, as_stream(stream));
 }
 
-extern "C" int rlse_gate_up_silu(const void* x, const void* w_gate_up, void* act, int rows,
-                                 int hidden, int inter, int dtype, void* workspace,
-                                 size_t workspace_bytes, rlse_stream_t stream) {
+static int gate_up_silu(const char* what, const Norm& norm, const void* x, const void* w_gate_up,
+                        void* act, int rows, int hidden, int inter, int dtype, void* workspace,
+                        size_t workspace_bytes, rlse_stream_t stream) {
   DenseParams flags{};
   take_packed(dtype, flags);
   const void* outs[1] = {act};
-  int rc = check_dense("gate_up_silu", dtype, rows, hidden, x, w_gate_up, outs, 1);
+  int rc = check_dense(what, dtype, rows, hidden, x, w_gate_up, outs, 1);
   if (rc || rows == 0) return rc;
+  rc = check_norm(what, norm, flags);
+  if (rc) return rc;
   if (inter <= 0 || inter % 8)
     return fail(RLSE_ERR_INVALID_VALUE,
-                "gate_up_silu: intermediate size %d must be a positive multiple of 8", inter);
+                "%s: intermediate size %d must be a positive multiple of 8", what, inter);
   if (flags.opacked && (inter % 32 || !aligned(act, 16)))
     return fail(RLSE_ERR_INVALID_VALUE,
-                "gate_up_silu: packed act needs inter a multiple of 32 (%d) and 16-byte alignment",
+                "%s: packed act needs inter a multiple of 32 (%d) and 16-byte alignment", what,
                 inter);
   DenseParams p{};
   p.x = x;
@@ -1135,10 +1317,26 @@ extern "C" int rlse_gate_up_silu(const void* x, const void* w_gate_up, void* act
   p.packed = flags.packed;
   p.xpacked = flags.xpacked;
   p.opacked = flags.opacked;
+  norm.set(p);
   size_t words = 0;
-  rc = dense_workspace("gate_up_silu", p, workspace, workspace_bytes, &words);
+  rc = dense_workspace(what, p, workspace, workspace_bytes, &words);
   if (rc) return rc;
   return dense_by_dtype<kEpiSiluMul>(dtype, p, words, as_stream(stream));
+}
+
+extern "C" int rlse_gate_up_silu(const void* x, const void* w_gate_up, void* act, int rows,
+                                 int hidden, int inter, int dtype, void* workspace,
+                                 size_t workspace_bytes, rlse_stream_t stream) {
+  return gate_up_silu("gate_up_silu", Norm{}, x, w_gate_up, act, rows, hidden, inter, dtype,
+                      workspace, workspace_bytes, stream);
+}
+
+extern "C" int rlse_norm_gate_up_silu(const void* residual, const void* norm_weight, float eps,
+                                      void* h, const void* w_gate_up, void* act, int rows,
+                                      int hidden, int inter, int dtype, void* workspace,
+                                      size_t workspace_bytes, rlse_stream_t stream) {
+  return gate_up_silu("norm_gate_up_silu", Norm{true, norm_weight, h, eps}, residual, w_gate_up,
+                      act, rows, hidden, inter, dtype, workspace, workspace_bytes, stream);
 }
 
 extern "C" int rlse_dense_pack(const void* weight, void* packed, int out_features,

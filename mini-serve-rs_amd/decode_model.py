@@ -12,16 +12,15 @@ seq_lens[b] - 1 (bf16 / f16: the projections on the MFMA kernels, fused with
 their neighbours):
 
     x = embed_tokens[ids]                                  rlse_embedding
-    h = input_layernorm(x)                                 rlse_add_rmsnorm (no add)
     the step's decode plan (page ids per wave)             rlse_decode_plan
     per layer:
-      q, k, v = q/k/v_proj(h)                              rlse_qkv_proj (one launch)
+      q, k, v = q/k/v_proj(input_layernorm(x))             rlse_norm_qkv_proj
       attn = q/k norm + RoPE + append + paged GQA decode    rlse_decode_step_planned
       x += o_proj(attn)                                    rlse_linear_residual
-      h = post_attention_layernorm(x)                      rlse_add_rmsnorm (no add)
-      a = silu(gate_proj(h)) * up_proj(h)                  rlse_gate_up_silu
+      h = post_attention_layernorm(x)
+      a = silu(gate_proj(h)) * up_proj(h)                  rlse_norm_gate_up_silu
       x += down_proj(a)                                    rlse_linear_residual
-      h = next input_layernorm(x) (the final norm last)    rlse_add_rmsnorm (no add)
+    h = norm(x)                                            rlse_add_rmsnorm (no add)
     logits = lm_head(h); next = argmax(logits)             rlse_linear, rlse_argmax
 
 f32 (a parity dtype, not a performance one) runs the same math as separate
@@ -308,15 +307,16 @@ class DecodeModel:
         H, nq, nkv = cfg.hidden, cfg.heads * cfg.head_dim, cfg.kv_heads * cfg.head_dim
         inter = cfg.inter
         kv.embedding(ids, self.embed, self.x, batch, H, cfg.vocab, dt, stream)
-        kv.add_rmsnorm(None, self.x, self.layers[0]["in_norm"], self.h, batch, H, cfg.eps, dt,
-                       stream, packed_out=self.packed if cfg.layers else self.lm_packed)
+        if not self.fused or not cfg.layers:
+            kv.add_rmsnorm(None, self.x, self.layers[0]["in_norm"] if cfg.layers else self.norm,
+                           self.h, batch, H, cfg.eps, dt, stream, packed_out=self.lm_packed)
         kv.decode_plan(block_tables, seq_lens, batch, cfg.kv_heads, self.mbps, self.num_blocks,
                        self.plan, self.plan.numel(), stream)
         for l, L in enumerate(self.layers):
             if self.fused:
-                kv.qkv_proj(self.h, L["qkv_w"], L["qkv_b"], self.q, self.k, self.v, batch, H, nq,
-                            nkv, dt, self.dense_ws, stream, packed=self.packed,
-                            packed_x=self.packed)
+                kv.norm_qkv_proj(self.x, L["in_norm"], cfg.eps, self.h, L["qkv_w"], L["qkv_b"],
+                                 self.q, self.k, self.v, batch, H, nq, nkv, dt, self.dense_ws,
+                                 stream, packed=self.packed)
             else:
                 kv.linear(self.h, L["q_w"], L["q_b"], self.q, batch, nq, H, dt, stream)
                 kv.linear(self.h, L["k_w"], L["k_b"], self.k, batch, nkv, H, dt, stream)
@@ -329,23 +329,15 @@ class DecodeModel:
                                    self.scale, dt, self.plan, self.workspace,
                                    self.workspace.numel(), stream,
                                    stream_pages=self.stream_pages)
-            nxt = self.layers[l + 1]["in_norm"] if l + 1 < cfg.layers else self.norm
             if self.fused:
                 kv.linear_residual(self.attn, L["o_w"], self.x, batch, H, nq, dt, self.dense_ws,
                                    stream, packed=self.packed)
-                kv.add_rmsnorm(None, self.x, L["post_norm"], self.h, batch, H, cfg.eps, dt,
-                               stream, packed_out=self.packed)
-                kv.gate_up_silu(self.h, L["gate_up_w"], self.act, batch, H, inter, dt,
-                                self.dense_ws, stream, packed=self.packed, packed_x=self.packed,
-                                packed_out=self.act_packed)
+                kv.norm_gate_up_silu(self.x, L["post_norm"], cfg.eps, self.h, L["gate_up_w"],
+                                     self.act, batch, H, inter, dt, self.dense_ws, stream,
+                                     packed=self.packed, packed_out=self.act_packed)
                 kv.linear_residual(self.act, L["down_w"], self.x, batch, H, inter, dt,
                                    self.dense_ws, stream, packed=self.packed,
                                    packed_x=self.act_packed)
-                # lm_head reads the final norm packed only if it runs on the
-                # MFMA kernel (vocab a multiple of 16)
-                last = l + 1 == cfg.layers
-                kv.add_rmsnorm(None, self.x, nxt, self.h, batch, H, cfg.eps, dt, stream,
-                               packed_out=self.lm_packed if last else self.packed)
             else:
                 kv.linear(self.attn, L["o_w"], None, self.o, batch, H, nq, dt, stream)
                 kv.add_rmsnorm(self.o, self.x, L["post_norm"], self.h, batch, H, cfg.eps, dt,
@@ -354,7 +346,13 @@ class DecodeModel:
                           stream)
                 kv.silu_mul(self.gu, self.act, batch, inter, dt, stream)
                 kv.linear(self.act, L["down_w"], None, self.o, batch, H, inter, dt, stream)
+                nxt = self.layers[l + 1]["in_norm"] if l + 1 < cfg.layers else self.norm
                 kv.add_rmsnorm(self.o, self.x, nxt, self.h, batch, H, cfg.eps, dt, stream)
+        if self.fused and cfg.layers:
+            # lm_head reads the final norm packed only if it runs on the MFMA
+            # kernel (vocab a multiple of 16)
+            kv.add_rmsnorm(None, self.x, self.norm, self.h, batch, H, cfg.eps, dt, stream,
+                           packed_out=self.lm_packed)
         kv.linear(self.h, self.lm_head, None, self.logits, batch, cfg.vocab, H, dt, stream,
                   packed=self.lm_packed, packed_x=self.lm_packed)
         kv.argmax(self.logits, self.next_ids, batch, cfg.vocab, dt, self.arg_ws,

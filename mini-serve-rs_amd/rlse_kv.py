@@ -76,6 +76,7 @@ EXPORTED = (
     "rlse_st_prepare", "rlse_st_host", "rlse_st_upload", "rlse_st_mark_uploaded",
     "rlse_embedding", "rlse_add_rmsnorm", "rlse_silu_mul", "rlse_argmax", "rlse_linear",
     "rlse_argmax_workspace_size", "rlse_qkv_proj", "rlse_linear_residual", "rlse_gate_up_silu",
+    "rlse_norm_qkv_proj", "rlse_norm_gate_up_silu",
     "rlse_dense_workspace_size", "rlse_dense_pack", "rlse_decode_plan_size", "rlse_decode_plan",
     "rlse_decode_step_planned", "rlse_workspace_check", "rlse_set_merge_wait_ns",
     "rlse_decode_step_noalloc", "rlse_decode_prefix_size", "rlse_decode_plan_cascade",
@@ -273,6 +274,9 @@ _SIGS = {
     "rlse_qkv_proj": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _sz, _vp]),
     "rlse_linear_residual": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp, _sz, _vp]),
     "rlse_gate_up_silu": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp, _sz, _vp]),
+    "rlse_norm_qkv_proj": (_i, [_vp, _vp, ctypes.c_float] + [_vp] * 6 + [_i] * 5 + [_vp, _sz, _vp]),
+    "rlse_norm_gate_up_silu": (_i, [_vp, _vp, ctypes.c_float] + [_vp] * 3 + [_i] * 4 +
+                               [_vp, _sz, _vp]),
     "rlse_dense_pack": (_i, [_vp, _vp, _i, _i, _i, _i, _vp]),
     "rlse_workspace_check": (_i, [_vp, _vp, ctypes.POINTER(ctypes.c_uint)]),
     "rlse_decode_step_noalloc": (_i, [_vp, _vp, _vp, _vp, _vp, _f, _vp, _vp, _i, _vp, _vp, _vp,
@@ -1034,6 +1038,29 @@ def qkv_proj(x, w_qkv, b_qkv, q, k, v, rows: int, hidden: int, q_features: int,
     _check(load().rlse_qkv_proj(_ptr(x), _ptr(w_qkv), _ptr(b_qkv), _ptr(q), _ptr(k), _ptr(v),
                                 rows, hidden, q_features, kv_features,
                                 _dtp(dtype, packed, packed_x), wp, wb, _stream(stream)))
+
+
+def norm_qkv_proj(residual, norm_weight, eps: float, h, w_qkv, b_qkv, q, k, v, rows: int,
+                  hidden: int, q_features: int, kv_features: int, dtype, workspace=None,
+                  stream=None, packed: bool = False) -> None:
+    """add_rmsnorm(None, residual, norm_weight, h) then qkv_proj; h is scratch."""
+    wp, wb = _ws(workspace)
+    _check(load().rlse_norm_qkv_proj(_ptr(residual), _ptr(norm_weight), eps, _ptr(h), _ptr(w_qkv),
+                                     _ptr(b_qkv), _ptr(q), _ptr(k), _ptr(v), rows, hidden,
+                                     q_features, kv_features, _dtp(dtype, packed, False), wp, wb,
+                                     _stream(stream)))
+
+
+def norm_gate_up_silu(residual, norm_weight, eps: float, h, w_gate_up, act, rows: int,
+                      hidden: int, inter: int, dtype, workspace=None, stream=None,
+                      packed: bool = False, packed_out: bool = False) -> None:
+    """add_rmsnorm(None, residual, norm_weight, h) then gate_up_silu; h is scratch."""
+    wp, wb = _ws(workspace)
+    _check(load().rlse_norm_gate_up_silu(_ptr(residual), _ptr(norm_weight), eps, _ptr(h),
+                                         _ptr(w_gate_up), _ptr(act), rows, hidden, inter,
+                                         _dtp(dtype, packed, False) |
+                                         (PACKED_OUT if packed_out else 0), wp, wb,
+                                         _stream(stream)))
 
 
 def linear_residual(x, weight, residual, rows: int, out_features: int, in_features: int, dtype,

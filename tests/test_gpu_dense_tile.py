@@ -1,4 +1,5 @@
-"""The fused projections over more rows than a decode batch (prompts).
+"""The fused projections over more rows than a decode batch (prompts), and the
+norm + projection calls.
 
 Reference: the q/k/v, o, gate/up and down projections of the prefill branch
 (src/backends/qwen2.rs:153-175, 233-252). Shapes put the output on each tile
@@ -107,3 +108,64 @@ def test_prompt_projections_match_oracle(kv, dt, packed, rows, hidden, nq, nkv, 
         want = O.round_to(res + O.linear_ref(a, wd, None, dt), dt)
         _close("linear_residual", y[:rows], want, dt, 2)
         assert bool((y[rows:] == 7).all())
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("rows,hidden,nq,nkv,inter", [
+    (1, 896, 896, 128, 4864),    # the norm in both launches (q/k/v: 16 waves, 2 k steps each)
+    (16, 1024, 2048, 1024, 3072),  # 8 k steps a wave
+    (7, 992, 4096, 32, 4096),    # 31 k steps; gate/up two tiles a workgroup
+    (9, 32, 4096, 16, 2048),     # one k step: waves without any
+    (5, 1056, 4096, 16, 2048),   # 33 k steps: the norm as a launch of its own
+    (17, 1024, 2048, 1024, 3072),  # past its row count
+    (70, 96, 64, 16, 64),        # a prompt
+    (2, 8224, 64, 16, 32)])      # rows longer than the register-held norm's
+def test_norm_projections_match_two_calls(kv, dt, packed, rows, hidden, nq, nkv, inter):
+    """norm_qkv_proj and norm_gate_up_silu against add_rmsnorm and the
+    projection: the sum of squares may run in another order (one unit in the
+    last place of a few h elements, far below the result's rounding); an
+    infinite row gives NaN either way, a huge one (its sum overflows) the
+    projection of zeros, and the residual is left alone."""
+    rng = np.random.default_rng(rows + hidden)
+    r = lambda *s: O.round_to(rng.standard_normal(s) / np.sqrt(s[-1]), dt)  # noqa: E731
+    tiles = (rows + 15) // 16 * 16
+    x = _dev(O.round_to(3 * rng.standard_normal((rows, hidden)), dt), dt)
+    if rows > 4:
+        x[2] = 0
+        x[3, 5] = float("inf")
+        x[4] = 3.0e38 if dt == "bf16" else 6.0e4
+    nw = _dev(O.round_to(1 + 0.1 * rng.standard_normal(hidden), dt), dt)
+    z = lambda n: torch.zeros((tiles, n), dtype=_T[dt], device=DEV)  # noqa: E731
+
+    def weight(w, pair=0):
+        w = _dev(w, dt)
+        if not packed:
+            return w
+        out = torch.empty_like(w)
+        kv.dense_pack(w, out, w.shape[0], w.shape[1], pair, dt)
+        return out
+
+    def ws(n_out):
+        n = kv.dense_workspace_size(rows, n_out, hidden)
+        return torch.zeros(max(n, 4), dtype=torch.uint8, device=DEV)
+
+    w, wg = weight(r(nq + 2 * nkv, hidden)), weight(r(2 * inter, hidden), inter)
+    b = _dev(O.round_to(rng.standard_normal(nq + 2 * nkv), dt), dt)
+    keep, h = x.clone(), z(hidden)
+    kv.add_rmsnorm(None, x, nw, h, rows, hidden, 1e-6, dt)
+    want = [z(n)[:rows] for n in (nq, nkv, nkv)] + [z(inter)]
+    kv.qkv_proj(h, w, b, *want[:3], rows, hidden, nq, nkv, dt, ws(nq + 2 * nkv), packed=packed)
+    kv.gate_up_silu(h, wg, want[3], rows, hidden, inter, dt, ws(2 * inter), packed=packed)
+    got = [z(n)[:rows] for n in (nq, nkv, nkv)] + [z(inter)]
+    kv.norm_qkv_proj(x, nw, 1e-6, z(hidden), w, b, *got[:3], rows, hidden, nq, nkv, dt,
+                     ws(nq + 2 * nkv), packed=packed)
+    kv.norm_gate_up_silu(x, nw, 1e-6, z(hidden), wg, got[3], rows, hidden, inter, dt,
+                         ws(2 * inter), packed=packed)
+    torch.cuda.synchronize()
+    assert torch.equal(x, keep)
+    for name, a, c, n in zip(("q", "k", "v", "act"), got, want, (2, 2, 2, 6)):
+        a, c = a[:rows].float().cpu().numpy(), c[:rows].float().cpu().numpy()
+        np.testing.assert_array_equal(np.isnan(a), np.isnan(c))
+        ok = ~np.isnan(c).any(1)
+        _close(name, a[ok], c[ok], dt, n)
