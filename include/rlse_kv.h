@@ -529,9 +529,9 @@ int rlse_linear(const void* x, const void* weight, const void* bias, void* y, in
 int rlse_dense_pack(const void* weight, void* packed, int out_features, int in_features,
                     int gate_up_inter, int dtype, rlse_stream_t stream);
 /* The three calls below are the decode step's projections fused with their
- * neighbours on MFMA (bf16/f16; in_features a multiple of 32; any rows --
- * up to 64 on a kernel shaped for a decode batch, more on one tiled for
- * prompts; x and weights 16-byte, outputs 8-byte aligned).
+ * neighbours on MFMA (bf16/f16; in_features a multiple of 32; any rows, and
+ * a row has the same bits whatever rows share its call; x and weights
+ * 16-byte, outputs 8-byte aligned).
  * workspace may be NULL; with rlse_dense_workspace_size bytes (for the
  * call's rows, total output features and in_features; zero-filled once
  * before its first use, then left to the library: error flags, launch

@@ -738,14 +738,13 @@ int dense_split(int groups, int K) {
 
 // Whether more than kDenseMaxRows rows still run on dense_rows_kernel (a
 // split that fits in the workgroup, a row tile per workgroup row) instead of
-// the tiled kernel: products with a long K and few output tiles, whose K the
-// 16 waves of a workgroup stream faster than one tile's pipeline. Measured
-// (us, here / tiled): 1024 x 3072 at 128 rows 7.8 / 8.8, at 256 rows 13.6 /
-// 9.3; 896 x 4864 at 128 rows 9.4 / 12.1, at 256 rows 17.0 / 12.9; with K
-// 2048, 1024 features and 128 rows 9.2 / 7.8.
-bool dense_long_k(int groups, int rows, int K) {
-  return K >= 96 * 32 && groups * ((rows + 15) / 16) <= 512;
-}
+// the tiled kernel: the same bits either way, and up to two workgroups per
+// compute unit the 16 waves of each stream K faster than one tile's
+// pipeline. Measured (us, here / tiled): 1024 x 2048 at 128 rows 6.5 / 8.4, at
+// 192 rows 8.8 / 8.6; 1024 x 3072 7.6 / 10.5 and 10.4 / 10.7; 896 x 4864 9.3 /
+// 14.5 and 13.3 / 14.8; 896 x 896 5.5 / 5.8 and 7.4 / 5.9; 1152 x 896 at 80
+// rows 5.6 / 5.8, at 128 rows 7.7 / 5.8; 3584 x 18944 at 80 rows 96.9 / 62.7.
+bool dense_few_tiles(int groups, int rows) { return groups * ((rows + 15LL) / 16) <= 512; }
 
 // Whether the norm before a product runs in its launch: every wave must hold
 // its k steps of x (8, or 2 in a 16-wave workgroup) and every workgroup all of
@@ -799,16 +798,18 @@ int launch_dense(DenseParams p, size_t ws_words, hipStream_t s) {
     p.norm_w = nullptr;
     return launch_dense<T, EPI>(p, ws_words, s);
   }
-  if constexpr (EPI != kEpiStore) {  // plain stores come 64 rows at a time
-    if (p.rows > kDenseMaxRows && !(kv_inner > 1 && dense_long_k(groups, p.rows, p.K)))
-      return launch_dense_tile(EPI, std::is_same<T, bf16>::value ? RLSE_DTYPE_BF16 : RLSE_DTYPE_F16,
-                               p, s);
-  }
   const int ns = kv_inner > 1 ? kv_inner : ks;
   const int steps_total = p.K / dense_step_elems<T>();
   const int slice = (steps_total + ns - 1) / ns;
   p.ksplit = kv_inner > 1 ? 1 : ks;
   p.steps = (slice + kDenseWaves - 1) / kDenseWaves;
+  if constexpr (EPI != kEpiStore) {  // plain stores come 64 rows at a time
+    if (p.rows > kDenseMaxRows && !(kv_inner > 1 && dense_few_tiles(groups, p.rows))) {
+      p.ksplit = ns;
+      return launch_dense_tile(EPI, std::is_same<T, bf16>::value ? RLSE_DTYPE_BF16 : RLSE_DTYPE_F16,
+                               p, s);
+    }
+  }
   const int rt = (p.rows + 15) / 16;
   if (p.ksplit > 1 && dense_ws_fixed_words() + (size_t)groups * (ks - 1) * ft * rt * 256 * 2 >
                           ws_words)

@@ -169,3 +169,57 @@ def test_norm_projections_match_two_calls(kv, dt, packed, rows, hidden, nq, nkv,
         np.testing.assert_array_equal(np.isnan(a), np.isnan(c))
         ok = ~np.isnan(c).any(1)
         _close(name, a[ok], c[ok], dt, n)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("kind,rows,n,k", [
+    ("qkv", 333, 4096, 1024),       # one slice of K: 64 x 64 tiles
+    ("qkv", 700, 4096, 992),        # 128 x 64 tiles, segments of 8, 8, 8 and 7 k steps
+    ("gate_up", 70, 8192, 32),      # one k step: the second half of K is empty
+    ("gate_up", 129, 8192, 160),    # 5 k steps in segments of 2
+    ("residual", 200, 2048, 1056),  # two slices
+    ("qkv", 97, 1536, 1056),        # three, of 11 k steps
+    ("residual", 300, 1024, 2048),  # four
+    ("residual", 800, 3584, 544),   # two, 128 x 64 tiles
+    ("residual", 90, 1024, 3072),   # four, few tiles
+    ("gate_up", 130, 640, 1024),    # seven, 32 x 32 tiles
+    ("gate_up", 150, 512, 1056)])   # eight
+@pytest.mark.parametrize("workspace", [True, False])
+def test_prompt_rows_have_the_bits_of_smaller_calls(kv, dt, kind, rows, n, k, workspace):
+    """Every row of a prompt's projections is, bit for bit, what a call of at
+    most 64 rows gives it (one token's K and V do not depend on the length of
+    the chunk it came in), with and without a K split, packed or not."""
+    g = torch.Generator(device=DEV).manual_seed(rows + n)
+    rnd = lambda *s: torch.randn(s, generator=g, device=DEV).to(_T[dt])  # noqa: E731
+    w, bias, res = rnd(n, k), rnd(n), rnd(rows, n)
+    x = rnd(rows, k)
+    n2 = 128 if n <= 1536 else 1024
+    packed = torch.empty_like(w)
+    kv.dense_pack(w, packed, n, k, n // 2 if kind == "gate_up" else 0, dt)
+    tiles = (rows + 15) // 16 * 16
+    px = torch.zeros((tiles, k), dtype=_T[dt], device=DEV)
+    px[:rows] = x
+    px = px.reshape(-1, 16, k // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous().reshape(tiles, k)
+
+    def call(x, res, r, w, packed, packed_x):
+        ws = torch.zeros(max(kv.dense_workspace_size(r, n, k), 8), dtype=torch.uint8, device=DEV)
+        ws = ws if workspace else None
+        flags = {"packed": packed, "packed_x": packed_x}
+        if kind == "qkv":
+            outs = [torch.empty((r, c), dtype=_T[dt], device=DEV) for c in (n - 2 * n2, n2, n2)]
+            kv.qkv_proj(x, w, bias, *outs, r, k, n - 2 * n2, n2, dt, ws, **flags)
+        elif kind == "residual":
+            outs = [res.clone()]
+            kv.linear_residual(x, w, outs[0], r, n, k, dt, ws, **flags)
+        else:
+            outs = [torch.empty((r, n // 2), dtype=_T[dt], device=DEV)]
+            kv.gate_up_silu(x, w, outs[0], r, k, n // 2, dt, ws, **flags)
+        return outs
+
+    chunks = [call(x[i:i + 64], res[i:i + 64], min(64, rows - i), w, False, False)
+              for i in range(0, rows, 64)]
+    want = [torch.cat(c) for c in zip(*chunks)]
+    for got in (call(x, res, rows, w, False, False), call(px, res, rows, packed, True, True)):
+        torch.cuda.synchronize()
+        for a, b in zip(got, want):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16))
