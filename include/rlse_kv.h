@@ -563,7 +563,8 @@ int rlse_gate_up_silu(const void* x, const void* w_gate_up, void* act, int rows,
 /* input_layernorm + q/k/v_proj and post_attention_layernorm + the MLP front
  * of the decode step (qwen2.rs:668-679, 750-753): rlse_add_rmsnorm(NULL,
  * residual, norm_weight, h) followed by rlse_qkv_proj / rlse_gate_up_silu on
- * h, in one launch for a decode batch of up to 16 rows whose shape allows it.
+ * h, to the bit; in one launch for a decode batch of up to 16 rows with hidden
+ * at most 1024 (gate/up, and q/k/v with few features, have further limits).
  * residual is row-major and only read; h (whole 16-row tiles) is scratch,
  * its contents afterwards unspecified. */
 int rlse_norm_qkv_proj(const void* residual, const void* norm_weight, float eps, void* h,

@@ -292,6 +292,23 @@ constexpr int kDenseMaxInner = 4;
 // when it has fewer than 256 tile groups, into ceil(256 / groups) slices.
 constexpr int kDenseCtrWords = 512 * kDenseWaves;
 constexpr int kDenseHeaderWords = 64;
+// Most k steps of a row whose norm runs in a projection's launch.
+constexpr int kNormSteps = 32;
+typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+
+// Lane groups of N of a and b interleaved, each with the sum of two: group 2i
+// holds a's groups 2i and 2i + 1, group 2i + 1 b's (a == b: a's in both).
+template <int N>
+__device__ __forceinline__ float add_swapped(float a, float b) {
+  const uint32_t x = __float_as_uint(a), z = __float_as_uint(b);
+  if constexpr (N == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(x, z, false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  } else {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, z, false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+}
 
 // KV > 1: the K split runs inside the workgroup instead of across
 // workgroups -- KV slices of kDenseWaves waves each, every wave on the k
@@ -300,11 +317,12 @@ constexpr int kDenseHeaderWords = 64;
 // order, then the slices in order), so the results are the split grid's to
 // the bit. No records, no launch counters, no second round trip to memory.
 //
-// NU > 0: x is the raw residual stream (row-major) and its RMSNorm runs here,
-// in place of a launch of norm_rows_kernel before: a wave holds all its k
-// steps (at most NU) of x and of the weights, the waves' sums of squares meet
-// in LDS while the weights are on their way, and each wave normalises its
-// own operands in registers, rounded as norm_rows_kernel rounds them.
+// NU > 0: x is the raw residual stream (row-major, at most kNormSteps k steps)
+// and its RMSNorm runs here, in place of a launch of norm_rows_kernel before:
+// a wave holds all its k steps (at most NU) of x and of the weights, the
+// steps' sums of squares meet in LDS while the weights are on their way, and
+// each wave normalises its own operands in registers, to norm_rows_kernel's
+// bits.
 template <typename T, int RT, int FT, int EPI, int KV = 1, int NU = 0>
 __global__ __launch_bounds__(64 * kDenseWaves * KV) void dense_rows_kernel(DenseParams p) {
   constexpr int WV = kDenseWaves * KV;  // waves per workgroup
@@ -420,23 +438,21 @@ __global__ __launch_bounds__(64 * kDenseWaves * KV) void dense_rows_kernel(Dense
   const int s_begin = sl * S / NS + ws * p.steps;
   const int s_end = min(slice_end, s_begin + p.steps);
   if constexpr (NU > 0) {
+    static_assert(RT == 1, "one row tile");
     // Every load is unconditional (steps past the wave's last re-read it and
     // are not used), so the waits below count loads and x is worked on while
     // the weights arrive.
-    __shared__ float s_ss[WV][RT][16];
+    __shared__ __align__(16) float s_ss[16][kNormSteps + 4];
     u32x4_t a[NU][FT], b[NU][RT], nw[NU];
     const int last = s_end > s_begin ? s_end - 1 : S - 1;
 #pragma unroll
-    for (int j = 0; j < NU; ++j) {
-      const int s = min(s_begin + j, last);
-#pragma unroll
-      for (int t = 0; t < RT; ++t)
-        b[j][t] = *reinterpret_cast<const u32x4_t*>(xr[t] + (size_t)xstep * s);
-    }
+    for (int j = 0; j < NU; ++j)
+      b[j][0] = *reinterpret_cast<const u32x4_t*>(xr[0] + (size_t)xstep * min(s_begin + j, last));
 #pragma unroll
     for (int j = 0; j < NU; ++j)
       nw[j] = *reinterpret_cast<const u32x4_t*>((const T*)p.norm_w + SE * min(s_begin + j, last) +
                                                 (SE / 4) * g);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < NU; ++j)
 #pragma unroll
@@ -444,45 +460,82 @@ __global__ __launch_bounds__(64 * kDenseWaves * KV) void dense_rows_kernel(Dense
         a[j][f] = *reinterpret_cast<const u32x4_t*>(wr[f] +
                                                     (size_t)wstep * min(s_begin + j, last));
     __builtin_amdgcn_sched_barrier(0);
+    // norm_rows_kernel's sum of squares: packets of 8 in element order, a
+    // balanced tree over 64 packets (16 k steps), its waves in order.
+    for (int i = threadIdx.x; i < 16 * kNormSteps; i += 64 * WV)
+      if (i / 16 >= S) s_ss[i % 16][i / 16] = 0.f;
+    u16x2_t least = 0xffff;  // least |h| of the wave's elements but zeros, as 2 * bits - 1
+    float part[NU];
 #pragma unroll
-    for (int t = 0; t < RT; ++t) {
-      float ss = 0.f;
+    for (int j = 0; j < NU; ++j) {
+      float h[8];
+      Packet<T>::unpack(__builtin_bit_cast(uint4, b[j][0]), h);
+      part[j] = 0.f;
 #pragma unroll
-      for (int j = 0; j < NU; ++j) {
-        float h[8], part = 0.f;
-        Packet<T>::unpack(__builtin_bit_cast(uint4, b[j][t]), h);
+      for (int e = 0; e < 8; ++e) part[j] += h[e] * h[e];
+      if constexpr (std::is_same<T, bf16>::value)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) part = fmaf(h[e], h[e], part);
-        ss += s_begin + j < s_end ? part : 0.f;
-      }
-      ss += __shfl_xor(ss, 16, 64);
-      ss += __shfl_xor(ss, 32, 64);
-      if (g == 0) s_ss[wave][t][fi] = ss;
+        for (int e = 0; e < 4; ++e) {
+          const u16x2_t u = __builtin_bit_cast(u16x2_t, b[j][0][e]);
+          least = __builtin_elementwise_min(least, (u16x2_t)(u * (uint16_t)2 - (uint16_t)1));
+        }
+    }
+    // The four packets of a step are in lanes fi + 16 g: each swap exchanges
+    // half of two steps' values, so lane group g ends with step 4 m + g of four.
+#pragma unroll
+    for (int m = 0; m < NU; m += 4) {
+      const float lo = add_swapped<16>(part[m], part[m + 1]);
+      const float hi = NU > 2 ? add_swapped<16>(part[m + 2], part[m + 3]) : lo;
+      const float sum = add_swapped<32>(lo, hi);
+      if (s_begin + m + g < s_end && g < NU) s_ss[fi][s_begin + m + g] = sum;
     }
     // A barrier for LDS alone: the weights stay in flight.
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const float4 q0 = *reinterpret_cast<const float4*>(&s_ss[fi][8 * g]);
+    const float4 q1 = *reinterpret_cast<const float4*>(&s_ss[fi][8 * g + 4]);
+    float ss = ((q0.x + q0.y) + (q0.z + q0.w)) + ((q1.x + q1.y) + (q1.z + q1.w));
+    ss += __shfl_xor(ss, 16, 64);
+    ss += __shfl_xor(ss, 32, 64);
+    const float norm = sqrtf(ss * p.inv_k + p.eps);
+    auto normalise = [&](uint4 hp, uint4 wp, auto divide) __attribute__((always_inline)) {
+      float h[8], w[8];
+      Packet<T>::unpack(hp, h);
+      Packet<T>::unpack(wp, w);
 #pragma unroll
-    for (int t = 0; t < RT; ++t) {
-      float ss = 0.f;
+      for (int e = 0; e < 8; ++e) h[e] = divide(h[e]);
+      Packet<T>::unpack(cvt_packet<T>(h), h);
 #pragma unroll
-      for (int w = 0; w < WV; ++w) ss += s_ss[w][t][fi];
-      // h / norm as the rounded reciprocal's product and one correction of its
-      // remainder, which rounds as the division does; an overflowed sum gives
-      // 0, as h / inf.
-      float norm = sqrtf(ss * p.inv_k + p.eps);
-      const float y = 1.f / norm;
-      norm = y == 0.f ? 0.f : norm;
+      for (int e = 0; e < 8; ++e) h[e] *= w[e];
+      return __builtin_bit_cast(u32x4_t, cvt_packet<T>(h));
+    };
+    // h / norm as the rounded reciprocal's product and one correction of its
+    // remainder: the rounded quotient for every 8- and 11-bit significand of h
+    // and every significand of norm (tests/test_quotient.py compares all
+    // pairs), where neither the quotient nor the remainder leaves the normal
+    // range.
+    const float y = 1.f / norm;
+#pragma unroll
+    for (int j = 0; j < NU; ++j)
+      b[j][0] = normalise(__builtin_bit_cast(uint4, b[j][0]), __builtin_bit_cast(uint4, nw[j]),
+                          [&](float h) {
+                            const float q = h * y;
+                            return fmaf(fmaf(-q, norm, h), y, q);
+                          });
+    // Where they might, or the sum overflowed or is zero: the division itself,
+    // of the row read again (kept for this, it would not fit the registers).
+    // Whole step, Qwen2.5-0.5B, one user: 987 us; with divisions alone 1049.
+    const bool plain = norm >= 0x1p-60f && norm <= 0x1p60f &&
+                       least[0] >= 0x42ff && least[1] >= 0x42ff;  // |h| >= 2^-60
+    if (__builtin_expect(!__all(plain), 0)) {
+      asm volatile("" ::: "memory");
 #pragma unroll
       for (int j = 0; j < NU; ++j) {
-        float h[8], w[8], o[8];
-        Packet<T>::unpack(__builtin_bit_cast(uint4, b[j][t]), h);
-        Packet<T>::unpack(__builtin_bit_cast(uint4, nw[j]), w);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float q = h[e] * y;
-          o[e] = round_cvt<T>(fmaf(fmaf(-q, norm, h[e]), y, q)) * w[e];
-        }
-        b[j][t] = __builtin_bit_cast(u32x4_t, cvt_packet<T>(o));
+        const int st = min(s_begin + j, last);
+        b[j][0] = normalise(*reinterpret_cast<const uint4*>(xr[0] + (size_t)xstep * st),
+                            *reinterpret_cast<const uint4*>((const T*)p.norm_w + SE * st +
+                                                            (SE / 4) * g),
+                            [&](float h) { return h / norm; });
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
 #pragma unroll
@@ -748,17 +801,17 @@ bool dense_few_tiles(int groups, int rows) { return groups * ((rows + 15LL) / 16
 
 // Whether the norm before a product runs in its launch: every wave must hold
 // its k steps of x (8, or 2 in a 16-wave workgroup) and every workgroup all of
-// K, for at most kDenseNormRows rows. A launch costs about 4 us between two
-// others, the norm of one row tile about 1 us of VALU time in each workgroup:
-// whole steps, Qwen2.5-0.5B, one user: 1022 -> 968 us; with two row tiles
-// (Qwen3-0.6B, 32 users) the step took 1849 against 1780 us.
+// K (hidden sizes to 1024: registers), for at most kDenseNormRows rows. A
+// launch costs about 4 us between two others, the norm of one row tile over 1 us
+// of VALU time in each workgroup: whole steps, Qwen2.5-0.5B, one user: 1031 ->
+// 987 us; with two row tiles (Qwen3-0.6B, 32 users) the step took 1849 against
+// 1780 us. The bits are the same either way.
 constexpr int kDenseNormRows = 16;
 template <int EPI>
 bool dense_norm_fits(const DenseParams& p, int ft, int ks, int kv_inner) {
   if ((EPI != kEpiQkv && EPI != kEpiSiluMul) || p.rows > kDenseNormRows || ft != 1) return false;
-  const int steps = p.K / 32;
-  if (kv_inner > 1) return EPI == kEpiQkv && kv_inner == 4 && ((steps + 3) / 4 + kDenseWaves - 1) / kDenseWaves <= 2;
-  return ks == 1 && (steps + kDenseWaves - 1) / kDenseWaves <= 8;
+  if (p.K / 32 > kNormSteps) return false;  // 8 k steps a wave of 4, 2 of 16
+  return kv_inner > 1 ? EPI == kEpiQkv && kv_inner == 4 : ks == 1;
 }
 
 // Launches a product: dense_rows_kernel for a decode batch, the tiled kernel
@@ -830,7 +883,7 @@ int launch_dense(DenseParams p, size_t ws_words, hipStream_t s) {
           }
         }
         // Two tiles a workgroup where 256 such groups are left: each norms
-        // the rows for itself (Qwen2.5-0.5B, one user, whole step 979 -> 968 us).
+        // the rows for itself (Qwen2.5-0.5B, one user, whole step 998 -> 987 us).
         if (tiles % 2 == 0 && tiles / 2 >= 256)
           hipLaunchKernelGGL((dense_rows_kernel<T, RT, 2, EPI, 1, 8>), dim3(tiles / 2), block, 0,
                              s, p);

@@ -223,3 +223,62 @@ def test_prompt_rows_have_the_bits_of_smaller_calls(kv, dt, kind, rows, n, k, wo
         torch.cuda.synchronize()
         for a, b in zip(got, want):
             assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("eps", [1e-6, 0.0])
+@pytest.mark.parametrize("hidden,nq,nkv,inter", [
+    (896, 896, 128, 4864),     # q/k/v: 16 waves, 2 k steps each; gate/up: two tiles a workgroup
+    (1024, 2048, 1024, 3072),  # 8 k steps a wave
+    (544, 4096, 32, 2048),     # 17 k steps: one past the first tree of 16
+    (32, 4096, 16, 2048),      # one
+    (1056, 4096, 16, 2048)])   # 33: the norm as a launch of its own at any row count
+def test_norm_projections_have_the_two_calls_bits(kv, dt, eps, hidden, nq, nkv, inter):
+    """norm_qkv_proj and norm_gate_up_silu give add_rmsnorm's and the
+    projection's bits, so a row's do not depend on whether its call norms in the
+    projection's launch (up to 16 rows) or before it: ordinary rows, rows with
+    elements far below the rest, rows whose squares underflow (with eps 0 the
+    division is by zero: infinities and NaN, not one for the other) or
+    overflow, and zeros."""
+    g = torch.Generator(device=DEV).manual_seed(hidden + nq)
+    rnd = lambda *s: torch.randn(s, generator=g, device=DEV)  # noqa: E731
+    x = 3 * rnd(33, hidden)
+    small = 1e-30 if dt == "bf16" else 6e-8
+    x[1] *= small
+    x[2, ::3] = small
+    x[3] = 0
+    x[4, 5 % hidden] = float("inf")
+    x[5] = 3.0e38 if dt == "bf16" else 6.0e4
+    x[6, ::2] *= 1e-38
+    x[7] *= 1e-20
+    x[8, 7] = float("nan")
+    x[9] = x[9].abs() * small  # with w[0] positive: an infinite product, not NaN
+    x = x.to(_T[dt])
+    nw = (1 + 0.1 * rnd(hidden)).to(_T[dt])
+    w, b = rnd(nq + 2 * nkv, hidden).to(_T[dt]), rnd(nq + 2 * nkv).to(_T[dt])
+    w[0] = w[0].abs() + 0.01
+    wg = rnd(2 * inter, hidden).to(_T[dt])
+
+    def call(lo, rows, fused):
+        xr, pad = x[lo:lo + rows].contiguous(), (rows + 15) // 16 * 16
+        h = torch.zeros((pad, hidden), dtype=_T[dt], device=DEV)
+        outs = [torch.zeros((rows, n), dtype=_T[dt], device=DEV) for n in (nq, nkv, nkv, inter)]
+        ws = [torch.zeros(max(kv.dense_workspace_size(rows, n, hidden), 8), dtype=torch.uint8,
+                          device=DEV) for n in (nq + 2 * nkv, 2 * inter)]
+        if fused:
+            kv.norm_qkv_proj(xr, nw, eps, h, w, b, *outs[:3], rows, hidden, nq, nkv, dt, ws[0])
+            kv.norm_gate_up_silu(xr, nw, eps, h, wg, outs[3], rows, hidden, inter, dt, ws[1])
+        else:
+            kv.add_rmsnorm(None, xr, nw, h, rows, hidden, eps, dt)
+            kv.qkv_proj(h, w, b, *outs[:3], rows, hidden, nq, nkv, dt, ws[0])
+            kv.gate_up_silu(h, wg, outs[3], rows, hidden, inter, dt, ws[1])
+        torch.cuda.synchronize()
+        return outs
+
+    want = call(0, 33, False)
+    for lo, rows in ((0, 1), (0, 7), (0, 16), (1, 16), (5, 1), (20, 13), (0, 17), (0, 33)):
+        for a, c in zip(call(lo, rows, True), want):
+            c = c[lo:lo + rows]
+            ok = ~c.isnan()
+            assert torch.equal(~a.isnan(), ok), (lo, rows)
+            assert torch.equal(a.view(torch.int16)[ok], c.view(torch.int16)[ok]), (lo, rows)
