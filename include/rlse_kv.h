@@ -380,9 +380,13 @@ int rlse_decode_step_noalloc(const void* q, const void* k_new, const void* v_new
  * pages with ids outside [0, num_blocks) are skipped. out [num_tokens]
  * [num_heads][head_dim]. f32, bf16 or f16 (MFMA tiles: f32 products for
  * f32, the reference CPU path's dtype), head_dim 64 or 128. workspace:
- * rlse_prefill_workspace_size bytes (may be 0), or NULL
- * for a library-owned one per device. Calls that share a workspace, the
- * library-owned one included, must be ordered (same stream). */
+ * rlse_prefill_workspace_size bytes (may be 0; enough for every call with no
+ * more tokens and no longer a context, in any dtype), or NULL for a
+ * library-owned one per device. The keys are split over workgroups only as far as the workspace holds
+ * the partial sums: a smaller one costs time, and is an error only where a
+ * context over 16384 keys has to be split. Calls
+ * that share a workspace, the library-owned one included, must be ordered
+ * (same stream). */
 int rlse_prefill_workspace_size(int num_tokens, int ctx_len, int num_heads, int num_kv_heads,
                                 int head_dim, size_t* bytes);
 int rlse_prefill_attn(const void* q, const void* k_pool, const void* v_pool,

@@ -755,11 +755,35 @@ __global__ __launch_bounds__(kPThreads) void prefill_merge_kernel(PrefillParams 
 // Workspace (key splits only): the partial blocks of every workgroup.
 struct PrefillPlan {
   int row_tiles, part_tiles, key_groups, splits, split_keys;
-  size_t ws_bytes;
 };
 
+size_t part_block_bytes(int D) { return (size_t)(4 * (D / 32) + 1) * kPThreads * 4 * sizeof(float); }
+
+// Fewest splits (a split's page ids must fit the LDS stage) and most.
+constexpr int kMaxSplitTiles = kMaxSplitPages * 16 / kBN;
+int min_splits(int ctx_len) {
+  return ((ctx_len + kBN - 1) / kBN + kMaxSplitTiles - 1) / kMaxSplitTiles;
+}
+int max_splits(int ctx_len) {
+  return std::min((ctx_len + kBN - 1) / kBN, std::max(kMaxSplits, min_splits(ctx_len)));
+}
+
+// The workspace of a call: what its largest plan can use, up to two partial
+// blocks per compute unit (71 MB at d = 128) or what the fewest splits of a
+// context over 16384 keys need. It grows with either length, so that one
+// sized for the longest chunk and context holds for every call. Plans with
+// more blocks would gain only for f32 chunks of 1100 to 1800 tokens (up to
+// 1.3 times by the estimate below; they run where a caller passes the memory).
+size_t prefill_ws_bytes(int Tq, int ctx_len, int Hq, int Hkv, int D, int cus) {
+  const long long tiles = (long long)((Tq * (Hq / Hkv) + kBM - 1) / kBM) * Hkv;
+  const int lo = min_splits(ctx_len), hi = max_splits(ctx_len);
+  const long long least = lo > 1 ? tiles * lo : 0, most = hi > 1 ? tiles * hi : 0;
+  return (size_t)std::max(least, std::min(most, 2LL * cus)) * part_block_bytes(D);
+}
+
 // Key groups of a workgroup and splits of the keys: the pair with the least
-// estimated time, in us,
+// estimated time among those whose partial blocks fit ws_bytes (at least the
+// fewest splits' must), in us,
 //   rounds of workgroups over the compute units x steps per split x t
 //   + (two key groups) 15% a step and the exchange
 //   + (more than one split) the merge launch, a round trip per kMergeBatch
@@ -775,26 +799,23 @@ struct PrefillPlan {
 // keys each: f32, 16/8 heads of 128, 333 tokens after 1030: 8 splits for 3,
 // 135 -> 68 us; 20 tokens after 1030: 17 for 3, 97 -> 22 us; bf16, 14/2 heads of
 // 64, 2000 tokens: 2 for 3 (one round for two), 36 -> 33 us.
-int plan_prefill(int Tq, int ctx_len, int Hq, int Hkv, int D, int dtype, PrefillPlan* plan) {
-  int cus = 0;
-  const int st = device_cu_count(&cus);
-  if (st) return st;
+bool plan_prefill(int Tq, int ctx_len, int Hq, int Hkv, int D, int dtype, int cus,
+                  size_t ws_bytes, PrefillPlan* plan) {
   const int G = Hq / Hkv;
   const int rows = Tq * G;
   plan->part_tiles = (rows + kBM - 1) / kBM;
-  const size_t block = (size_t)(4 * (D / 32) + 1) * kPThreads * 4 * sizeof(float);
+  const size_t block = part_block_bytes(D);
   const double tile_us = dtype == RLSE_DTYPE_F32 ? (D == 128 ? 14.7 : 7.7) : (D == 128 ? 1.9 : 1.2);
   const int tiles = (ctx_len + kBN - 1) / kBN;
-  const int most = kMaxSplitPages * 16 / kBN;  // a split's page ids must fit the LDS stage
-  const int limit = std::min(tiles, std::max(kMaxSplits, (tiles + most - 1) / most));
   double best_us = 0.;
   plan->splits = 0;
   for (int kg = 1; kg <= (dtype != RLSE_DTYPE_F32 && D == 128 ? 2 : 1); ++kg) {
     const int row_tiles = (rows + kBM / kg - 1) / (kBM / kg);
     const long long base = (long long)row_tiles * Hkv;
-    for (int want = 1; want <= limit; ++want) {
+    for (int want = min_splits(ctx_len); want <= max_splits(ctx_len); ++want) {
       const int per = (tiles + want - 1) / want, s = (tiles + per - 1) / per;
-      if (s != want || per > most) continue;  // (fewer splits gave the same shares)
+      if (s != want) continue;  // (fewer splits gave the same shares)
+      if (s > 1 && (size_t)s * plan->part_tiles * Hkv * block > ws_bytes) break;
       if (kg > 1 && per <= 2) continue;
       const int steps = (per + kg - 1) / kg;
       double us = (double)((base * s + cus - 1) / cus) * steps * tile_us;
@@ -810,8 +831,7 @@ int plan_prefill(int Tq, int ctx_len, int Hq, int Hkv, int D, int dtype, Prefill
       }
     }
   }
-  plan->ws_bytes = plan->splits > 1 ? (size_t)plan->splits * plan->part_tiles * Hkv * block : 0;
-  return RLSE_OK;
+  return plan->splits > 0;
 }
 
 template <typename T, int D>
@@ -885,14 +905,10 @@ extern "C" int rlse_prefill_workspace_size(int num_tokens, int ctx_len, int num_
   if (num_tokens <= 0 || ctx_len < num_tokens || num_heads <= 0 || num_kv_heads <= 0 ||
       num_heads % num_kv_heads != 0 || (head_dim != 64 && head_dim != 128))
     return fail(RLSE_ERR_INVALID_VALUE, "prefill_workspace_size: bad shape");
-  // The dtype is not known here: what either element size needs.
-  PrefillPlan p16, p32;
-  int st = plan_prefill(num_tokens, ctx_len, num_heads, num_kv_heads, head_dim, RLSE_DTYPE_BF16,
-                        &p16);
-  if (!st)
-    st = plan_prefill(num_tokens, ctx_len, num_heads, num_kv_heads, head_dim, RLSE_DTYPE_F32, &p32);
+  int cus = 0;
+  const int st = device_cu_count(&cus);
   if (st) return st;
-  *bytes = std::max(p16.ws_bytes, p32.ws_bytes);
+  *bytes = prefill_ws_bytes(num_tokens, ctx_len, num_heads, num_kv_heads, head_dim, cus);
   return RLSE_OK;
 }
 
@@ -908,30 +924,36 @@ extern "C" int rlse_prefill_attn(const void* q, const void* k_pool, const void* 
     return fail(RLSE_ERR_INVALID_VALUE, "prefill: null pointer argument");
   if (!(scale > 0.f) || !isfinite(scale))
     return fail(RLSE_ERR_INVALID_VALUE, "prefill: scale must be finite and positive");
-  PrefillPlan plan;
-  st = plan_prefill(num_tokens, ctx_len, num_heads, num_kv_heads, head_dim, dtype, &plan);
+  int cus = 0;
+  st = device_cu_count(&cus);
   if (st) return st;
+  const hipStream_t s = as_stream(stream);
   std::unique_lock<std::mutex> lock;
-  if (plan.ws_bytes > 0) {
-    if (workspace == nullptr) {
-      int dev = 0;
-      hipError_t e = hipGetDevice(&dev);
-      if (e != hipSuccess || dev < 0 || dev >= 64)
+  int dev = 0;
+  if (workspace == nullptr) {
+    workspace_bytes = prefill_ws_bytes(num_tokens, ctx_len, num_heads, num_kv_heads, head_dim, cus);
+    if (workspace_bytes > 0) {
+      if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
         return fail(RLSE_ERR_INVALID_VALUE, "prefill: no current device");
       lock = std::unique_lock<std::mutex>(g_pws_mu);
-      if (g_pws_size[dev] < plan.ws_bytes) {
-        if (g_pws_ptr[dev]) (void)hipFree(g_pws_ptr[dev]);
-        g_pws_ptr[dev] = nullptr;
-        g_pws_size[dev] = 0;
-        e = hipMalloc(&g_pws_ptr[dev], plan.ws_bytes);
-        if (e != hipSuccess) return fail((int)e, "prefill: workspace hipMalloc failed");
-        g_pws_size[dev] = plan.ws_bytes;
-      }
-      workspace = g_pws_ptr[dev];
-    } else if (workspace_bytes < plan.ws_bytes) {
-      return fail(RLSE_ERR_BUFFER_TOO_SMALL, "prefill: workspace %zu bytes < %zu needed",
-                  workspace_bytes, plan.ws_bytes);
     }
+  }
+  PrefillPlan plan;
+  if (!plan_prefill(num_tokens, ctx_len, num_heads, num_kv_heads, head_dim, dtype, cus,
+                    workspace_bytes, &plan))
+    return fail(RLSE_ERR_BUFFER_TOO_SMALL, "prefill: workspace %zu bytes < %zu needed",
+                workspace_bytes, (size_t)min_splits(ctx_len) * plan.part_tiles * num_kv_heads *
+                                     part_block_bytes(head_dim));
+  if (plan.splits > 1 && workspace == nullptr) {
+    if (g_pws_size[dev] < workspace_bytes) {
+      if (g_pws_ptr[dev]) (void)hipFree(g_pws_ptr[dev]);
+      g_pws_ptr[dev] = nullptr;
+      g_pws_size[dev] = 0;
+      const hipError_t e = hipMalloc(&g_pws_ptr[dev], workspace_bytes);
+      if (e != hipSuccess) return fail((int)e, "prefill: workspace hipMalloc failed");
+      g_pws_size[dev] = workspace_bytes;
+    }
+    workspace = g_pws_ptr[dev];
   }
   PrefillParams pp{};
   pp.q = q;
@@ -953,11 +975,12 @@ extern "C" int rlse_prefill_attn(const void* q, const void* k_pool, const void* 
   pp.splits = plan.splits;
   pp.split_keys = plan.split_keys;
   pp.c = scale * 1.4426950408889634f;
-  const hipStream_t s = as_stream(stream);
+  const int kg = plan.key_groups;
   if (dtype == RLSE_DTYPE_BF16)
-    return head_dim == 128 ? launch_prefill<bf16, 128>(pp, plan.key_groups, s) : launch_prefill<bf16, 64>(pp, plan.key_groups, s);
+    return head_dim == 128 ? launch_prefill<bf16, 128>(pp, kg, s)
+                           : launch_prefill<bf16, 64>(pp, kg, s);
   if (dtype == RLSE_DTYPE_F32)
-    return head_dim == 128 ? launch_prefill<float, 128>(pp, plan.key_groups, s)
-                           : launch_prefill<float, 64>(pp, plan.key_groups, s);
-  return head_dim == 128 ? launch_prefill<f16, 128>(pp, plan.key_groups, s) : launch_prefill<f16, 64>(pp, plan.key_groups, s);
+    return head_dim == 128 ? launch_prefill<float, 128>(pp, kg, s)
+                           : launch_prefill<float, 64>(pp, kg, s);
+  return head_dim == 128 ? launch_prefill<f16, 128>(pp, kg, s) : launch_prefill<f16, 64>(pp, kg, s);
 }

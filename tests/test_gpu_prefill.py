@@ -17,7 +17,7 @@ import pytest
 import torch
 
 import oracle as O
-from gpu_helpers import TOL, as_f32, err_report, random_values, to_dev, to_host
+from gpu_helpers import DEV, TOL, as_f32, err_report, random_values, to_dev, to_host
 
 pytestmark = pytest.mark.gpu
 
@@ -212,3 +212,45 @@ def test_prefill_row_and_key_groups_match_oracle(kv, dtype, hq, hkv, d, tq, offs
     mx, rel = err_report(got, want)
     print(f"[prefill groups {hq}/{hkv}/{d} {tq}+{offset}] {dtype} max_abs={mx:.3e} rel={rel:.3e}")
     assert np.isfinite(got).all() and mx <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype,hq,hkv,d,large,small", [
+    ("f32", 16, 8, 128, (256, 1280), (200, 1000)),
+    ("bf16", 28, 4, 128, (2048, 2048), (200, 1000)),
+    ("bf16", 14, 2, 64, (2048, 2100), (64, 1500)),
+    ("f16", 32, 8, 128, (512, 17000), (5, 9000))])
+def test_prefill_workspace_holds_for_smaller_calls(kv, dtype, hq, hkv, d, large, small):
+    """A workspace sized once for the longest chunk and context is enough for
+    every smaller call, and the size never falls with either length."""
+    size = kv.prefill_workspace_size(*large, hq, hkv, d)
+    for tq in (1, 7, 64, 200, 500, 1000, 1667, 2048):
+        for ctx in (2048, 2100, 9743, 17000, 40000):
+            n = kv.prefill_workspace_size(tq, ctx, hq, hkv, d)
+            assert n >= kv.prefill_workspace_size(tq, max(tq, ctx - 900), hq, hkv, d)
+            assert n >= kv.prefill_workspace_size(max(1, tq // 2), ctx, hq, hkv, d)
+            # two blocks of 256 rows (f32 sums and a max and a sum) per compute unit, or
+            # the splits that page ids in LDS ask for
+            tiles = -(-tq * (hq // hkv) // 256) * hkv
+            assert n <= max(512, -(-ctx // 16384) * tiles) * 256 * (d + 8) * 4
+    rng = np.random.default_rng(hq + d)
+    tq, L = small
+    q, kp, vp, table, L = make_case(rng, hq, hkv, d, tq, L - tq, dtype)
+    scale = 1.0 / math.sqrt(d)
+    want = oracle_prefill(q, kp, vp, table, L, hq, hkv, d, dtype, scale)
+    qd, kd, vd, td = to_dev(q, dtype), to_dev(kp, dtype), to_dev(vp, dtype), to_dev(table)
+    for n in (size, size // 8, 0):
+        ws = torch.empty(max(n, 16), dtype=torch.uint8, device=DEV)
+        out = torch.empty_like(qd)
+        kv.prefill_attn(qd, kd, vd, td, L, tq, out, hq, hkv, d, len(table), kp.shape[0], scale,
+                        dtype, ws, n)
+        torch.cuda.synchronize()
+        check(f"prefill workspace {n}", as_f32(to_host(out), dtype), want, dtype)
+
+
+def test_prefill_long_context_needs_its_workspace(kv):
+    """Over 16384 keys must be split: a workspace too small for that is refused."""
+    d = torch.zeros(64, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(kv.RlseError) as e:
+        kv.prefill_attn(d, d, d, torch.zeros(1025, dtype=torch.int32, device=DEV), 16390, 1, d, 4,
+                        1, 128, 1025, 1, 0.1, "bf16", d, d.numel() * 2)
+    assert e.value.status == kv.ERR_BUFFER_TOO_SMALL
