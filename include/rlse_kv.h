@@ -382,7 +382,8 @@ int rlse_decode_step_noalloc(const void* q, const void* k_new, const void* v_new
  * f32, the reference CPU path's dtype), head_dim 64 or 128. workspace:
  * rlse_prefill_workspace_size bytes (may be 0; enough for every call with no
  * more tokens and no longer a context, in any dtype), or NULL for a
- * library-owned one per device. The keys are split over workgroups only as far as the workspace holds
+ * library-owned one per device (which a call in a stream capture uses as it
+ * is). The keys are split over workgroups only as far as the workspace holds
  * the partial sums: a smaller one costs time, and is an error only where a
  * context over 16384 keys has to be split. Calls
  * that share a workspace, the library-owned one included, must be ordered

@@ -936,6 +936,11 @@ extern "C" int rlse_prefill_attn(const void* q, const void* k_pool, const void* 
       if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
         return fail(RLSE_ERR_INVALID_VALUE, "prefill: no current device");
       lock = std::unique_lock<std::mutex>(g_pws_mu);
+      // Nothing can be allocated into a capture: it runs in what is there.
+      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+      if (g_pws_size[dev] < workspace_bytes &&
+          hipStreamIsCapturing(s, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone)
+        workspace_bytes = g_pws_size[dev];
     }
   }
   PrefillPlan plan;

@@ -10,7 +10,10 @@ Bars: max-abs 2e-2 for bf16 and f16 (the probabilities enter the P.V product
 rounded to the pool dtype), 2e-3 for f32 (the reference CPU path's dtype: f32
 products on f32 MFMAs); the relative error is printed beside it.
 """
+import importlib.util
 import math
+import shutil
+import sys
 
 import numpy as np
 import pytest
@@ -254,3 +257,39 @@ def test_prefill_long_context_needs_its_workspace(kv):
         kv.prefill_attn(d, d, d, torch.zeros(1025, dtype=torch.int32, device=DEV), 16390, 1, d, 4,
                         1, 128, 1025, 1, 0.1, "bf16", d, d.numel() * 2)
     assert e.value.status == kv.ERR_BUFFER_TOO_SMALL
+
+
+def test_prefill_captured_before_any_workspace_exists(kv, tmp_path, monkeypatch):
+    """A chunk short enough to run unsplit can be captured with the
+    library-owned workspace although nothing has allocated one yet (a copy of
+    the library has its own); every replay gives the eager result's values."""
+    lib = tmp_path / "librlse_kv_copy.so"
+    shutil.copy(kv.LIB_PATH, lib)
+    monkeypatch.setenv("RLSE_KV_LIB", str(lib))
+    spec = importlib.util.spec_from_file_location("rlse_kv_copy", kv.__file__)
+    fresh = importlib.util.module_from_spec(spec)
+    monkeypatch.setitem(sys.modules, "rlse_kv_copy", fresh)
+    spec.loader.exec_module(fresh)
+    rng = np.random.default_rng(3)
+    hq, hkv, d, tq, dtype = 16, 8, 128, 20, "f32"
+    q, kp, vp, table, L = make_case(rng, hq, hkv, d, tq, 400, dtype)
+    scale = 1.0 / math.sqrt(d)
+    qd, kd, vd, td = to_dev(q), to_dev(kp), to_dev(vp), to_dev(table)
+    out = torch.empty_like(qd)
+
+    def call():
+        fresh.prefill_attn(qd, kd, vd, td, L, tq, out, hq, hkv, d, len(table), kp.shape[0], scale,
+                           dtype, stream=torch.cuda.current_stream())
+
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    want = oracle_prefill(q, kp, vp, table, L, hq, hkv, d, dtype, scale)
+    for _ in range(3):
+        out.fill_(7)
+        graph.replay()
+        torch.cuda.synchronize()
+        check("captured", to_host(out), want, dtype)
+        call()  # eager: allocates
+        torch.cuda.synchronize()
+        check("eager", to_host(out), want, dtype)
