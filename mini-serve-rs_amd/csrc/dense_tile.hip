@@ -412,35 +412,51 @@ __global__ __launch_bounds__(64 * kTWaves, 4) void dense_tile_kernel(TileParams 
   }
 }
 
+// A grid holds fewer than 2^32 threads: more tiles run as several launches.
+constexpr long long kMaxTiles = (1LL << 32) / (64 * kTWaves) - 8;
+
 template <typename T, int EPI, int BF, int BR, int NB>
 int run_tile(const DenseParams& p, hipStream_t s) {
   const int ntiles = EPI == kEpiSiluMul ? p.n1 / 8 : p.N / 16;
-  const int nfb = (ntiles * 16 + BF - 1) / BF, nrb = (p.rows + BR - 1) / BR;
-  const long long total = (long long)nfb * nrb;
-  if (total > (1LL << 28)) return fail(RLSE_ERR_INVALID_VALUE, "dense: too many rows");
-  const int per = (int)((total + 7) / 8);
-  // A run of band x (per / band) tiles reads band * BF + (per / band) * BR
-  // rows of the two operands: least at band = sqrt(per * BR / BF).
-  const int square = (int)(sqrt((double)per * BR / BF) + 0.5);
-  const int band = std::min(nfb, std::max(std::max(1, square), (per + nrb - 1) / nrb));
+  const int nfb = (int)((ntiles * 16LL + BF - 1) / BF);
+  if (nfb > kMaxTiles) return fail(RLSE_ERR_INVALID_VALUE, "dense: too many features");
   const int S = p.K / 32, n = p.ksplit;
   const int second = n > 3 ? 2 : 1, first = n - second;  // slices of the halves
   TileParams t;
-  t.x = p.x, t.w = p.w, t.bias = p.bias;
-  t.out0 = p.out0, t.out1 = p.out1, t.out2 = p.out2;
-  t.rows = p.rows, t.K = p.K, t.N = p.N, t.n1 = p.n1, t.n2 = p.n2;
-  t.ntiles = ntiles, t.nfb = nfb, t.nrb = nrb, t.band = band, t.per = per;
+  t.w = p.w, t.bias = p.bias;
+  t.K = p.K, t.N = p.N, t.n1 = p.n1, t.n2 = p.n2;
+  t.ntiles = ntiles, t.nfb = nfb;
   t.steps = p.steps, t.cut = n > 1 ? first * S / n : std::min(2 * p.steps, S);
   t.slices = n, t.q = S / n, t.r = S % n, t.rem = first * (S % n) % n;
   t.second = second;
   t.packed = p.packed, t.xpacked = p.xpacked, t.opacked = p.opacked;
-  if (n > 1)
-    hipLaunchKernelGGL((dense_tile_kernel<T, EPI, BF, BR, NB, true>), dim3(8 * per),
-                       dim3(64 * kTWaves), 0, s, t);
-  else
-    hipLaunchKernelGGL((dense_tile_kernel<T, EPI, BF, BR, NB, false>), dim3(8 * per),
-                       dim3(64 * kTWaves), 0, s, t);
-  return launch_status("dense_tile_kernel");
+  const long long max_rows = kMaxTiles / nfb * BR;
+  for (long long r0 = 0; r0 < p.rows; r0 += max_rows) {
+    const int rows = (int)std::min<long long>(p.rows - r0, max_rows);
+    const int nrb = (int)((rows + BR - 1LL) / BR);
+    const int per = (int)(((long long)nfb * nrb + 7) / 8);
+    // A run of band x (per / band) tiles reads band * BF + (per / band) * BR
+    // rows of the two operands: least at band = sqrt(per * BR / BF).
+    const int square = (int)(sqrt((double)per * BR / BF) + 0.5);
+    t.band = std::min(nfb, std::max(std::max(1, square), (per + nrb - 1) / nrb));
+    t.rows = rows, t.nrb = nrb, t.per = per;
+    // (Whole 16-row tiles: packed rows are as far apart as row-major ones.)
+    auto from = [&](const void* base, int features) {
+      return base ? (void*)((T*)base + (size_t)r0 * features) : nullptr;
+    };
+    t.x = from(p.x, p.K);
+    t.out0 = from(p.out0, EPI == kEpiResidual ? p.N : p.n1);
+    t.out1 = from(p.out1, p.n2 - p.n1), t.out2 = from(p.out2, p.N - p.n2);
+    if (n > 1)
+      hipLaunchKernelGGL((dense_tile_kernel<T, EPI, BF, BR, NB, true>), dim3(8 * per),
+                         dim3(64 * kTWaves), 0, s, t);
+    else
+      hipLaunchKernelGGL((dense_tile_kernel<T, EPI, BF, BR, NB, false>), dim3(8 * per),
+                         dim3(64 * kTWaves), 0, s, t);
+    const int rc = launch_status("dense_tile_kernel");
+    if (rc) return rc;
+  }
+  return RLSE_OK;
 }
 
 // The tile shape, by how many workgroups each makes of the output. A larger

@@ -282,3 +282,24 @@ def test_norm_projections_have_the_two_calls_bits(kv, dt, eps, hidden, nq, nkv, 
             ok = ~c.isnan()
             assert torch.equal(~a.isnan(), ok), (lo, rows)
             assert torch.equal(a.view(torch.int16)[ok], c.view(torch.int16)[ok]), (lo, rows)
+
+
+def test_more_rows_than_a_grid_holds(kv):
+    """2^23 row tiles of 512 threads pass the 2^32 threads of a grid: the rows
+    before, at and after that point, and the last, are those of small calls."""
+    rows, n, k, dt = (1 << 29) + 1000, 16, 32, "bf16"
+    g = torch.Generator(device=DEV).manual_seed(1)
+    w = torch.randn((n, k), generator=g, device=DEV).to(_T[dt])
+    x = torch.zeros((rows, k), dtype=_T[dt], device=DEV)
+    y = torch.zeros((rows, n), dtype=_T[dt], device=DEV)
+    spans = [(0, 300), ((1 << 29) - 1024, (1 << 29) + 300), (rows - 100, rows)]
+    for a, b in spans:
+        x[a:b] = torch.randn((b - a, k), generator=g, device=DEV).to(_T[dt])
+    kv.linear_residual(x, w, y, rows, n, k, dt)
+    for a, b in spans:
+        want = torch.zeros((b - a, n), dtype=_T[dt], device=DEV)
+        kv.linear_residual(x[a:b], w, want, b - a, n, k, dt)
+        torch.cuda.synchronize()
+        assert torch.equal(y[a:b], want) and bool(want.any(1).all())
+    del x, y
+    torch.cuda.empty_cache()
