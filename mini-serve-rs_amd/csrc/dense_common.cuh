@@ -11,16 +11,16 @@ typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 template <typename T>
-struct Mma16;
+struct DenseMma;
 template <>
-struct Mma16<bf16> {
+struct DenseMma<bf16> {
   static __device__ __forceinline__ f32x4_t run(u32x4_t a, u32x4_t b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
                                                    __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
   }
 };
 template <>
-struct Mma16<f16> {
+struct DenseMma<f16> {
   static __device__ __forceinline__ f32x4_t run(u32x4_t a, u32x4_t b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
                                                   __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
@@ -33,7 +33,7 @@ struct Mma16<f16> {
 // the lane groups g, and the four products cover the step. The accumulator
 // layout is the 16-bit products' (lane l: D[4*(l/16) + v][l%16]).
 template <>
-struct Mma16<float> {
+struct DenseMma<float> {
   static __device__ __forceinline__ f32x4_t run(u32x4_t a, u32x4_t b, f32x4_t c) {
 #pragma unroll
     for (int m = 0; m < 4; ++m)

@@ -267,7 +267,7 @@ __global__ __launch_bounds__(64 * kTWaves, 4) void dense_tile_kernel(TileParams 
 #pragma unroll
     for (int f = 0; f < FT; ++f)
 #pragma unroll
-      for (int r = 0; r < RT; ++r) acc[f * RT + r] = Mma16<T>::run(a[f], b[r], acc[f * RT + r]);
+      for (int r = 0; r < RT; ++r) acc[f * RT + r] = DenseMma<T>::run(a[f], b[r], acc[f * RT + r]);
     __builtin_amdgcn_sched_barrier(0);
   };
   // The stages whose prefetch and steps exist in both halves, then the rest.

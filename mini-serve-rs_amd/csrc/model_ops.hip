@@ -544,7 +544,7 @@ __global__ __launch_bounds__(64 * kDenseWaves * KV) void dense_rows_kernel(Dense
 #pragma unroll
         for (int f = 0; f < FT; ++f)
 #pragma unroll
-          for (int t = 0; t < RT; ++t) acc[f][t] = Mma16<T>::run(a[j][f], b[j][t], acc[f][t]);
+          for (int t = 0; t < RT; ++t) acc[f][t] = DenseMma<T>::run(a[j][f], b[j][t], acc[f][t]);
       }
   }
   for (int s = s_begin; NU == 0 && s < s_end; s += U) {
@@ -566,7 +566,7 @@ __global__ __launch_bounds__(64 * kDenseWaves * KV) void dense_rows_kernel(Dense
 #pragma unroll
         for (int f = 0; f < FT; ++f)
 #pragma unroll
-          for (int t = 0; t < RT; ++t) acc[f][t] = Mma16<T>::run(a[j][f], b[j][t], acc[f][t]);
+          for (int t = 0; t < RT; ++t) acc[f][t] = DenseMma<T>::run(a[j][f], b[j][t], acc[f][t]);
       }
     }
   }

@@ -100,3 +100,16 @@ def test_rope_tables_match_oracle(kv, orc):
     cb, _ = kv.rope_tables(1e6, 128, 700, kv.DTYPE_BF16)
     np.testing.assert_array_equal(np.frombuffer(cb, np.uint16).reshape(700, 64),
                                   orc.f32_to_bf16_bits(oc))
+
+
+def test_headers_define_each_name_once():
+    """The device headers share one named namespace: a class of the same name
+    in two of them would be two definitions of one class in the library."""
+    csrc = os.path.join(ROOT, "mini-serve-rs_amd", "csrc")
+    seen = {}
+    for name in sorted(os.listdir(csrc)):
+        if name.endswith((".cuh", ".h")):
+            with open(os.path.join(csrc, name)) as f:
+                for cls in set(re.findall(r"^(?:struct|class|union) (\w+)\b(?!<)", f.read(), re.M)):
+                    assert cls not in seen, (cls, name, seen[cls])
+                    seen[cls] = name
