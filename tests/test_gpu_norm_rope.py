@@ -192,3 +192,38 @@ def test_qk_norm_rope_append_packet_rows_give_the_element_bits(kv, dtype, hq, hk
                     for t in (q_out, kp, vp)])
     for x, y in zip(*got):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_conversion_instruction_rounds_to_nearest_even(kv, dtype):
+    """Roundings through the conversion instruction (the projections'
+    epilogues, the norms, the q/k norm + RoPE) against the integer sequence: a
+    product whose f32 results are a 16-bit value plus each of the 2^16 lower
+    significands. Signs, exponents to the overflow and (f16) subnormal edges."""
+    tdt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    # x = [hi, 2^e, 2^e'] against w = [1, low / 256, low % 256]: sums of at most 24 significant
+    # bits, exact in f32 in any order.
+    low = torch.arange(1 << 16, device=DEV)
+    w = torch.zeros((1 << 16, 32), device=DEV)
+    w[:, 0], w[:, 1], w[:, 2] = 1, low // 256, low % 256
+    exps = (range(-100, 128, 9) if dtype == "bf16" else range(-18, 16))
+    rows = [(s * (1 + m / 128), e) for e in list(exps) + ([127] if dtype == "bf16" else [])
+            for m in (0, 1, 2, 63, 64, 127) for s in (1.0, -1.0)]
+    x = torch.zeros((len(rows), 32), dtype=torch.float64, device=DEV)
+    for i, (m, e) in enumerate(rows):
+        sign = 1 if m > 0 else -1
+        x[i, 0] = m * 2.0 ** e
+        x[i, 1], x[i, 2] = sign * 2.0 ** (e - 15), sign * 2.0 ** (e - 23)
+    keep = (x.to(tdt).double() == x).all(1)  # (f16 has no 2^(e - 23) for the smallest)
+    assert int(keep.sum()) >= 60
+    x = x[keep]
+    exact = (x @ w.double().T).float()  # one f32 each
+    bits = exact.view(torch.int32)
+    if dtype == "bf16":
+        want = ((bits + 0x7FFF + ((bits >> 16) & 1)) >> 16).to(torch.int16)
+    else:
+        want = exact.cpu().half().view(torch.int16).to(DEV)
+    out = torch.zeros((x.shape[0], 1 << 16), dtype=tdt, device=DEV)
+    kv.linear(x.to(tdt).contiguous(), w.to(tdt), None, out, x.shape[0], 1 << 16, 32, dtype)
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), want)

@@ -140,6 +140,41 @@ def test_prefill_skips_invalid_pages(kv, dtype):
     check("invalid pages skipped", got, want, dtype)
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("hq,hkv,tq,offset", [
+    (16, 8, 32, 200),    # two key groups, one split; spare waves only stage
+    (16, 8, 200, 200),   # the full kernel
+    (4, 1, 3, 2000),     # eight splits
+    (4, 1, 150, 4100)])  # twelve, of three steps each
+@pytest.mark.parametrize("bad", ["even", "odd", "all even", "all odd", "each in turn"])
+def test_prefill_key_groups_skip_invalid_pages(kv, dtype, hq, hkv, tq, offset, bad):
+    """Two key groups take the even and the odd 64-key tiles of a step: page
+    ids outside the pool in the tiles of one group only, on every page of that
+    group (its keys are all masked) or at another place in each tile hide the
+    same keys as a float64 evaluation without them."""
+    d = 128
+    rng = np.random.default_rng(tq + offset)
+    q, kp, vp, table, L = make_case(rng, hq, hkv, d, tq, offset, dtype)
+    scale = 1 / math.sqrt(d)
+    page = np.arange(len(table))
+    odd, at = page // 4 % 2 == 1, page % 4
+    hit = {"even": ~odd & (at == 1), "odd": odd & (at == 2), "all even": ~odd, "all odd": odd,
+           "each in turn": page % 8 == page // 8 % 8}[bad]
+    table_bad = table.copy()
+    table_bad[hit] = np.where(page[hit] % 3 == 0, -1, kp.shape[0] + page[hit]).astype(np.int32)
+    got = as_f32(run_prefill(kv, q, kp, vp, table_bad, L, hq, hkv, d, dtype, scale), dtype)
+    kc = as_f32(O.paged_to_contiguous(kp, table, L), dtype).astype(np.float64)
+    vc = as_f32(O.paged_to_contiguous(vp, table, L), dtype).astype(np.float64)
+    qf = as_f32(q, dtype).astype(np.float64)
+    visible = ~np.repeat(hit, 16)[:L] & (np.arange(L) <= offset + np.arange(tq)[:, None])
+    want = np.zeros_like(qf)
+    for hh in range(hq):
+        x = np.where(visible, qf[:, hh] @ kc[hh // (hq // hkv)].T * scale, -np.inf)
+        p = np.exp(x - x.max(1, keepdims=True))
+        want[:, hh] = p / p.sum(1, keepdims=True) @ vc[hh // (hq // hkv)]
+    check(f"invalid pages, {bad}", got, want, dtype)
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 def test_prefill_qwen3_8b_chunk(kv, dtype):
     """The Qwen3-8B chunk: 512 queries after 8192 cached tokens, 32 q / 8 kv
