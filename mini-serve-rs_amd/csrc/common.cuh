@@ -74,8 +74,9 @@ __device__ __forceinline__ float round_to(float v) {
   return Elem<T>::to_f32(Elem<T>::from_f32(v));
 }
 
-// round_to through the conversion instruction: the same bits for every input
-// (NaNs included) without the integer sequence of f32_to_bf16_bits.
+// round_to through the conversion instruction, without the integer sequence of
+// f32_to_bf16_bits: the same bits (the tests compare every lower half of a
+// float, ties, overflow and NaN rows).
 template <typename T>
 __device__ __forceinline__ float round_cvt(float v) {
   if constexpr (sizeof(T) == 4)

@@ -501,6 +501,7 @@ __device__ __forceinline__ uint16_t bits_sel(float v) {
     return u;
   }
 }
+
 // Packs EPL floats of a row slice into a 16-byte packet of T.
 template <typename T>
 __device__ __forceinline__ uint4 pack_packet(const float* y) {
@@ -525,7 +526,7 @@ __device__ __forceinline__ uint4 pack_packet(const float* y) {
 // of squares is sumsq_tree's order with one packet per lane, so every entry
 // point that writes K stores the same bytes. Roundings take the conversion
 // instruction: against the integer sequence, 64 forked sequences (28 layers)
-// 881 -> 844 us, Qwen2.5-0.5B's 64 x 4096 tokens 722 -> 714 us.
+// 881 -> 844 us; long contexts, where the rows are few, are as fast with either.
 template <typename T, int D>
 __device__ __forceinline__ uint4 norm_rope_packet(uint4 x, bool norm, uint4 w, float inv_d,
                                                   float eps, uint4 cs, uint4 sn, int col) {
@@ -1112,8 +1113,10 @@ __device__ __forceinline__ void decode_body(const DecodeParams& p,
             T* dst = ob + ((size_t)b * Hq + (size_t)kvh * G + mh) * D + 4 * mq;
 #pragma unroll
             for (int t = 0; t < D / 16; ++t) {
-              const uint32_t w0 = (uint32_t)bits_sel<T>(macc[t][0] * inv) | ((uint32_t)bits_sel<T>(macc[t][1] * inv) << 16);
-              const uint32_t w1 = (uint32_t)bits_sel<T>(macc[t][2] * inv) | ((uint32_t)bits_sel<T>(macc[t][3] * inv) << 16);
+              const uint32_t w0 = (uint32_t)bits_sel<T>(macc[t][0] * inv) |
+                                  ((uint32_t)bits_sel<T>(macc[t][1] * inv) << 16);
+              const uint32_t w1 = (uint32_t)bits_sel<T>(macc[t][2] * inv) |
+                                  ((uint32_t)bits_sel<T>(macc[t][3] * inv) << 16);
               *reinterpret_cast<uint2*>(dst + 16 * t) = make_uint2(w0, w1);
             }
           }

@@ -118,9 +118,9 @@ __device__ __forceinline__ float4* part_block(const PrefillParams& p, int sp, in
 }
 
 // FEW: a chunk too short to give every wave of the one row tile rows; the
-// waves without any then only stage. (Left out otherwise: the branch around
-// the math costs the full kernel 3-9%; with 5 tokens of a group of 4 it takes
-// 8000 cached keys from 28.6 to 21.7 us.)
+// waves without any then only stage: f32, 20 tokens after 1030, 28.5 -> 21.3
+// us; bf16, one token after 99, 6.9 -> 6.4, longer contexts as fast with either.
+// (Left out otherwise: the branch around the math costs the full kernel 3-9%.)
 template <typename T, int D, int KG, bool FEW>
 __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) {
   constexpr int KB = D / 16;                  // 16-wide k-blocks of q.k
@@ -275,86 +275,88 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel(PrefillParams p) 
       const int vbits = (s_valid[bf] >> (4 * kg)) & 15;
 
       if (!FEW || live) {
-      // S^T for the two 32-key halves of the tile.
-      // (The two halves' MFMA chains are interleaved: consecutive MFMAs then
-      // never wait on each other's accumulator.)
-      f32x16_t s[2];
-#pragma unroll
-      for (int sb = 0; sb < 2; ++sb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s[sb][i] = 0.f;
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-        for (int sb = 0; sb < 2; ++sb) {
-          const uint4 a =
-              *reinterpret_cast<const uint4*>(&s_k[bf][kBN * kg + sb * 32 + col][kb * 16 + half * 8]);
-          s[sb] = Mfma<T>::mma(a, qreg[kb], s[sb]);
-        }
-      // Mask (causal, past the split's end, invalid pages) only on tiles that
-      // need it: the test is wave-uniform and most tiles are fully visible.
-      if (!(kt + kBN - 1 <= kmin_wave && kt + kBN <= k_end && vbits == 15)) {
+        // S^T for the two 32-key halves of the tile.
+        // (The two halves' MFMA chains are interleaved: consecutive MFMAs then
+        // never wait on each other's accumulator.)
+        f32x16_t s[2];
 #pragma unroll
         for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int kk = sb * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-            const int ka = kt + kk;
-            if (!(ka <= kmax && ka < k_end && ((vbits >> (kk >> 4)) & 1))) s[sb][i] = -INFINITY;
+          for (int i = 0; i < 16; ++i) s[sb][i] = 0.f;
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+          for (int sb = 0; sb < 2; ++sb) {
+            const uint4 a =
+                *reinterpret_cast<const uint4*>(
+                    &s_k[bf][kBN * kg + sb * 32 + col][kb * 16 + half * 8]);
+            s[sb] = Mfma<T>::mma(a, qreg[kb], s[sb]);
           }
-      }
-      float mx = -INFINITY;
+        // Mask (causal, past the split's end, invalid pages) only on tiles that
+        // need it: the test is wave-uniform and most tiles are fully visible.
+        if (!(kt + kBN - 1 <= kmin_wave && kt + kBN <= k_end && vbits == 15)) {
 #pragma unroll
-      for (int sb = 0; sb < 2; ++sb)
+          for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[sb][i]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      // Online softmax in log2 units (the scale folded into the exponent's
-      // FMA). The running max moves only when a score exceeds it by more
-      // than kLazyLog2, so the accumulator rescale is rare.
-      const float cand = mx * p.c;
-      if (__any(cand > m + kLazyLog2)) {
-        const float mn = fmaxf(m, cand);
-        const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
-        lsum *= alpha;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
-        m = mn;
-      }
-      const float nms = m == -INFINITY ? 0.f : -m;
-      float rs = 0.f;
-      uint4 pk[4];  // P^T operands of the four 16-key blocks
-#pragma unroll
-      for (int sb = 0; sb < 2; ++sb) {
-        float pr[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          pr[i] = __builtin_amdgcn_exp2f(fmaf(s[sb][i], p.c, nms));
-          rs += pr[i];
+            for (int i = 0; i < 16; ++i) {
+              const int kk = sb * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
+              const int ka = kt + kk;
+              if (!(ka <= kmax && ka < k_end && ((vbits >> (kk >> 4)) & 1))) s[sb][i] = -INFINITY;
+            }
         }
+        float mx = -INFINITY;
 #pragma unroll
-        for (int kb2 = 0; kb2 < 2; ++kb2) {
-          const float* v8 = pr + kb2 * 8;
-          pk[sb * 2 + kb2] = make_uint4(Packet<T>::pack2(v8[0], v8[1]), Packet<T>::pack2(v8[2], v8[3]),
-                                        Packet<T>::pack2(v8[4], v8[5]), Packet<T>::pack2(v8[6], v8[7]));
+        for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[sb][i]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        // Online softmax in log2 units (the scale folded into the exponent's
+        // FMA). The running max moves only when a score exceeds it by more
+        // than kLazyLog2, so the accumulator rescale is rare.
+        const float cand = mx * p.c;
+        if (__any(cand > m + kLazyLog2)) {
+          const float mn = fmaxf(m, cand);
+          const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+          lsum *= alpha;
+#pragma unroll
+          for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
+          m = mn;
         }
-      }
-      rs += __shfl_xor(rs, 32, 64);
-      lsum += rs;
-      // O^T += V^T . P^T
+        const float nms = m == -INFINITY ? 0.f : -m;
+        float rs = 0.f;
+        uint4 pk[4];  // P^T operands of the four 16-key blocks
 #pragma unroll
-      for (int kq = 0; kq < 4; ++kq)
+        for (int sb = 0; sb < 2; ++sb) {
+          float pr[16];
 #pragma unroll
-        for (int db = 0; db < DB; ++db) {
-          const uint16_t* v0 = &s_v[bf][kBN * kg + kq * 16 + tr_row][db * 32 + tr_col];
-          const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)v0);
-          const i16x4_t hi =
-              __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(v0 + 8 * (D + kPadV)));
-          const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
-          o[db] = Mfma<T>::mma(make_uint4(l2.x, l2.y, h2.x, h2.y), pk[kq], o[db]);
+          for (int i = 0; i < 16; ++i) {
+            pr[i] = __builtin_amdgcn_exp2f(fmaf(s[sb][i], p.c, nms));
+            rs += pr[i];
+          }
+#pragma unroll
+          for (int kb2 = 0; kb2 < 2; ++kb2) {
+            const float* v8 = pr + kb2 * 8;
+            pk[sb * 2 + kb2] =
+                make_uint4(Packet<T>::pack2(v8[0], v8[1]), Packet<T>::pack2(v8[2], v8[3]),
+                           Packet<T>::pack2(v8[4], v8[5]), Packet<T>::pack2(v8[6], v8[7]));
+          }
         }
+        rs += __shfl_xor(rs, 32, 64);
+        lsum += rs;
+        // O^T += V^T . P^T
+#pragma unroll
+        for (int kq = 0; kq < 4; ++kq)
+#pragma unroll
+          for (int db = 0; db < DB; ++db) {
+            const uint16_t* v0 = &s_v[bf][kBN * kg + kq * 16 + tr_row][db * 32 + tr_col];
+            const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)v0);
+            const i16x4_t hi =
+                __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(v0 + 8 * (D + kPadV)));
+            const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+            o[db] = Mfma<T>::mma(make_uint4(l2.x, l2.y, h2.x, h2.y), pk[kq], o[db]);
+          }
       }
 
       if (!more) break;
@@ -577,70 +579,71 @@ __global__ __launch_bounds__(kPThreads, 1) void prefill_kernel_f32(PrefillParams
       const int vbits = s_valid[bf];
 
       if (!FEW || live) {
-      f32x16_t s[2];
+        f32x16_t s[2];
 #pragma unroll
-      for (int sb = 0; sb < 2; ++sb)
+        for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[sb][i] = 0.f;
+          for (int i = 0; i < 16; ++i) s[sb][i] = 0.f;
 #pragma unroll
-      for (int j = 0; j < KH; j += 4)
+        for (int j = 0; j < KH; j += 4)
 #pragma unroll
-        for (int sb = 0; sb < 2; ++sb) {
-          const float4 a = *reinterpret_cast<const float4*>(&s_k[bf][sb * 32 + col][half * KH + j]);
-          s[sb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, qreg[j], s[sb], 0, 0, 0);
-          s[sb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, qreg[j + 1], s[sb], 0, 0, 0);
-          s[sb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, qreg[j + 2], s[sb], 0, 0, 0);
-          s[sb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, qreg[j + 3], s[sb], 0, 0, 0);
+          for (int sb = 0; sb < 2; ++sb) {
+            const float4 a =
+                *reinterpret_cast<const float4*>(&s_k[bf][sb * 32 + col][half * KH + j]);
+            s[sb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, qreg[j], s[sb], 0, 0, 0);
+            s[sb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, qreg[j + 1], s[sb], 0, 0, 0);
+            s[sb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, qreg[j + 2], s[sb], 0, 0, 0);
+            s[sb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, qreg[j + 3], s[sb], 0, 0, 0);
+          }
+        if (!(kt + kBN - 1 <= kmin_wave && kt + kBN <= k_end && vbits == 15)) {
+#pragma unroll
+          for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const int kk = sb * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
+              const int ka = kt + kk;
+              if (!(ka <= kmax && ka < k_end && ((vbits >> (kk >> 4)) & 1))) s[sb][i] = -INFINITY;
+            }
         }
-      if (!(kt + kBN - 1 <= kmin_wave && kt + kBN <= k_end && vbits == 15)) {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[sb][i]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float cand = mx * p.c;
+        if (__any(cand > m + kLazyLog2)) {
+          const float mn = fmaxf(m, cand);
+          const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+          lsum *= alpha;
+#pragma unroll
+          for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
+          m = mn;
+        }
+        const float nms = m == -INFINITY ? 0.f : -m;
+        float rs = 0.f;
 #pragma unroll
         for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
-            const int kk = sb * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-            const int ka = kt + kk;
-            if (!(ka <= kmax && ka < k_end && ((vbits >> (kk >> 4)) & 1))) s[sb][i] = -INFINITY;
+            s[sb][i] = __builtin_amdgcn_exp2f(fmaf(s[sb][i], p.c, nms));
+            rs += s[sb][i];
           }
-      }
-      float mx = -INFINITY;
+        rs += __shfl_xor(rs, 32, 64);
+        lsum += rs;
+        // O^T += V^T . P^T, step j of key half sb: the lane's half takes key
+        // sb*32 + 8*(j/4) + 4*half + j%4 (its accumulator element j).
 #pragma unroll
-      for (int sb = 0; sb < 2; ++sb)
+        for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[sb][i]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float cand = mx * p.c;
-      if (__any(cand > m + kLazyLog2)) {
-        const float mn = fmaxf(m, cand);
-        const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
-        lsum *= alpha;
+          for (int j = 0; j < 16; ++j) {
+            const float* vrow = &s_v[bf][sb * 32 + (j >> 2) * 8 + half * 4 + (j & 3)][col];
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
-        m = mn;
-      }
-      const float nms = m == -INFINITY ? 0.f : -m;
-      float rs = 0.f;
-#pragma unroll
-      for (int sb = 0; sb < 2; ++sb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          s[sb][i] = __builtin_amdgcn_exp2f(fmaf(s[sb][i], p.c, nms));
-          rs += s[sb][i];
-        }
-      rs += __shfl_xor(rs, 32, 64);
-      lsum += rs;
-      // O^T += V^T . P^T, step j of key half sb: the lane's half takes key
-      // sb*32 + 8*(j/4) + 4*half + j%4 (its accumulator element j).
-#pragma unroll
-      for (int sb = 0; sb < 2; ++sb)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const float* vrow = &s_v[bf][sb * 32 + (j >> 2) * 8 + half * 4 + (j & 3)][col];
-#pragma unroll
-          for (int db = 0; db < DB; ++db)
-            o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[db * 32], s[sb][j], o[db], 0, 0, 0);
-        }
+            for (int db = 0; db < DB; ++db)
+              o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[db * 32], s[sb][j], o[db], 0, 0, 0);
+          }
       }
 
       if (!more) break;
@@ -757,7 +760,9 @@ struct PrefillPlan {
   int row_tiles, part_tiles, key_groups, splits, split_keys;
 };
 
-size_t part_block_bytes(int D) { return (size_t)(4 * (D / 32) + 1) * kPThreads * 4 * sizeof(float); }
+size_t part_block_bytes(int D) {
+  return (size_t)(4 * (D / 32) + 1) * kPThreads * 4 * sizeof(float);
+}
 
 // Fewest splits (a split's page ids must fit the LDS stage) and most.
 constexpr int kMaxSplitTiles = kMaxSplitPages * 16 / kBN;
@@ -772,8 +777,9 @@ int max_splits(int ctx_len) {
 // blocks per compute unit (71 MB at d = 128) or what the fewest splits of a
 // context over 16384 keys need. It grows with either length, so that one
 // sized for the longest chunk and context holds for every call. Plans with
-// more blocks would gain only for f32 chunks of 1100 to 1800 tokens (up to
-// 1.3 times by the estimate below; they run where a caller passes the memory).
+// more blocks gain only for f32 chunks of 1100 to 1800 tokens (1135 after 7101,
+// 32/8 heads: 1228 us in 134 MiB, 1346 in this, 2004 unsplit in one round of
+// workgroups); they run where a caller passes the memory.
 size_t prefill_ws_bytes(int Tq, int ctx_len, int Hq, int Hkv, int D, int cus) {
   const long long tiles = (long long)((Tq * (Hq / Hkv) + kBM - 1) / kBM) * Hkv;
   const int lo = min_splits(ctx_len), hi = max_splits(ctx_len);
