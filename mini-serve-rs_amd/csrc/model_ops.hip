@@ -258,7 +258,8 @@ __global__ __launch_bounds__(64) void argmax_final_kernel(const T* __restrict__ 
 // ---------------------------------------------------------------------------
 // Decode-shaped linear layers on MFMA: y[rows][N] = x[rows][K] . W[N][K]^T for
 // rows <= 64 (one decode step's batch; more run on the tiled kernel of
-// dense_tile.hip), bf16/f16 in, f32 accumulation.
+// dense_tile.hip, or here where there are few tiles), bf16/f16 in, f32
+// accumulation.
 //
 // Work split: workgroup (g, ks) owns FT tiles of 16 output features, the
 // whole batch and the ks-th of KS equal slices of K; its four waves split the
