@@ -323,9 +323,12 @@ __device__ __forceinline__ float add_swapped(float a, float b) {
 // a wave holds all its k steps (at most NU) of x and of the weights, the
 // steps' sums of squares meet in LDS while the weights are on their way, and
 // each wave normalises its own operands in registers, to norm_rows_kernel's
-// bits.
+// bits. (Two waves a SIMD at least, which keeps the accumulators out of AGPRs:
+// they were copied there and back at every branch around a k step that a wave
+// does not have.)
 template <typename T, int RT, int FT, int EPI, int KV = 1, int NU = 0>
-__global__ __launch_bounds__(64 * kDenseWaves * KV) void dense_rows_kernel(DenseParams p) {
+__global__ __launch_bounds__(64 * kDenseWaves * KV, NU > 0 ? 2 : 1) void dense_rows_kernel(
+    DenseParams p) {
   constexpr int WV = kDenseWaves * KV;  // waves per workgroup
   if constexpr (KV > 1 && RT == 1 && (EPI == kEpiResidual || EPI == kEpiQkv)) {
     // Row tiles split over the grid's rows (the launcher does so only for
@@ -524,7 +527,7 @@ __global__ __launch_bounds__(64 * kDenseWaves * KV) void dense_rows_kernel(Dense
                           });
     // Where they might, or the sum overflowed or is zero: the division itself,
     // of the row read again (kept for this, it would not fit the registers).
-    // Whole step, Qwen2.5-0.5B, one user: 987 us; with divisions alone 1049.
+    // Whole step, Qwen2.5-0.5B, one user: 985 us; with divisions alone 1037.
     const bool plain = norm >= 0x1p-60f && norm <= 0x1p60f &&
                        least[0] >= 0x42ff && least[1] >= 0x42ff;  // |h| >= 2^-60
     if (__builtin_expect(!__all(plain), 0)) {
@@ -804,8 +807,8 @@ bool dense_few_tiles(int groups, int rows) { return groups * ((rows + 15LL) / 16
 // its k steps of x (8, or 2 in a 16-wave workgroup) and every workgroup all of
 // K (hidden sizes to 1024: registers), for at most kDenseNormRows rows. A
 // launch costs about 4 us between two others, the norm of one row tile over 1 us
-// of VALU time in each workgroup: whole steps, Qwen2.5-0.5B, one user: 1031 ->
-// 987 us; with two row tiles (Qwen3-0.6B, 32 users) the step took 1849 against
+// of VALU time in each workgroup: whole steps, Qwen2.5-0.5B, one user: 1032 ->
+// 985 us; with two row tiles (Qwen3-0.6B, 32 users) the step took 1849 against
 // 1780 us. The bits are the same either way.
 constexpr int kDenseNormRows = 16;
 template <int EPI>
@@ -884,7 +887,7 @@ int launch_dense(DenseParams p, size_t ws_words, hipStream_t s) {
           }
         }
         // Two tiles a workgroup where 256 such groups are left: each norms
-        // the rows for itself (Qwen2.5-0.5B, one user, whole step 998 -> 987 us).
+        // the rows for itself (Qwen2.5-0.5B, one user, whole step 1004 -> 985 us).
         if (tiles % 2 == 0 && tiles / 2 >= 256)
           hipLaunchKernelGGL((dense_rows_kernel<T, RT, 2, EPI, 1, 8>), dim3(tiles / 2), block, 0,
                              s, p);
