@@ -934,38 +934,43 @@ extern "C" int rlse_prefill_attn(const void* q, const void* k_pool, const void* 
   st = device_cu_count(&cus);
   if (st) return st;
   const hipStream_t s = as_stream(stream);
-  std::unique_lock<std::mutex> lock;
-  int dev = 0;
-  if (workspace == nullptr) {
+  if (workspace == nullptr)
     workspace_bytes = prefill_ws_bytes(num_tokens, ctx_len, num_heads, num_kv_heads, head_dim, cus);
-    if (workspace_bytes > 0) {
-      if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
-        return fail(RLSE_ERR_INVALID_VALUE, "prefill: no current device");
-      lock = std::unique_lock<std::mutex>(g_pws_mu);
-      // Nothing can be allocated into a capture: it runs in what is there.
-      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-      if (g_pws_size[dev] < workspace_bytes &&
-          hipStreamIsCapturing(s, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone)
-        workspace_bytes = g_pws_size[dev];
-    }
-  }
   PrefillPlan plan;
-  if (!plan_prefill(num_tokens, ctx_len, num_heads, num_kv_heads, head_dim, dtype, cus,
-                    workspace_bytes, &plan))
-    return fail(RLSE_ERR_BUFFER_TOO_SMALL, "prefill: workspace %zu bytes < %zu needed",
-                workspace_bytes, (size_t)min_splits(ctx_len) * plan.part_tiles * num_kv_heads *
-                                     part_block_bytes(head_dim));
-  if (plan.splits > 1 && workspace == nullptr) {
+  auto plan_in = [&](size_t bytes) {
+    return plan_prefill(num_tokens, ctx_len, num_heads, num_kv_heads, head_dim, dtype, cus, bytes,
+                        &plan);
+  };
+  bool fits = plan_in(workspace_bytes);
+  std::unique_lock<std::mutex> lock;
+  if (workspace == nullptr && plan.splits > 1) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
+      return fail(RLSE_ERR_INVALID_VALUE, "prefill: no current device");
+    lock = std::unique_lock<std::mutex>(g_pws_mu);
     if (g_pws_size[dev] < workspace_bytes) {
-      if (g_pws_ptr[dev]) (void)hipFree(g_pws_ptr[dev]);
-      g_pws_ptr[dev] = nullptr;
-      g_pws_size[dev] = 0;
-      const hipError_t e = hipMalloc(&g_pws_ptr[dev], workspace_bytes);
-      if (e != hipSuccess) return fail((int)e, "prefill: workspace hipMalloc failed");
-      g_pws_size[dev] = workspace_bytes;
+      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+      hipError_t e = hipStreamIsCapturing(s, &capture);
+      if (e != hipSuccess) return fail((int)e, "prefill: hipStreamIsCapturing failed");
+      if (capture != hipStreamCaptureStatusNone) {
+        // Nothing can be allocated into a capture: it runs in what is there.
+        workspace_bytes = g_pws_size[dev];
+        fits = plan_in(workspace_bytes);
+      } else {
+        if (g_pws_ptr[dev]) (void)hipFree(g_pws_ptr[dev]);
+        g_pws_ptr[dev] = nullptr;
+        g_pws_size[dev] = 0;
+        e = hipMalloc(&g_pws_ptr[dev], workspace_bytes);
+        if (e != hipSuccess) return fail((int)e, "prefill: workspace hipMalloc failed");
+        g_pws_size[dev] = workspace_bytes;
+      }
     }
     workspace = g_pws_ptr[dev];
   }
+  if (!fits)
+    return fail(RLSE_ERR_BUFFER_TOO_SMALL, "prefill: workspace %zu bytes < %zu needed",
+                workspace_bytes, (size_t)min_splits(ctx_len) * plan.part_tiles * num_kv_heads *
+                                     part_block_bytes(head_dim));
   PrefillParams pp{};
   pp.q = q;
   pp.k_pool = k_pool;
